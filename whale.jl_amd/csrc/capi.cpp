@@ -70,16 +70,12 @@ hipError_t upload(DBuf& b, const std::vector<T>& v, hipStream_t st) {
 
 struct whale_batch;
 namespace {
-// The searchable launch shape of a batch.
 constexpr int kLayouts = 6;
-// Layout kLayoutPool: no size classes; one pooled launch (k_pool) runs every
-// family whose stages fit LDS, its forward and reverse sweep by one wave with
-// LDS pages taken from its compute unit's pool.
-constexpr int kLayoutPool = kLayouts;
+// The searchable launch shape of a batch.
 struct Tuning {
-  uint32_t bounds[5] = {10 * 1024, 14 * 1024, 20 * 1024, 28 * 1024, 48 * 1024};  // class LDS bounds (bytes)
-  int layout = 0;      // index into kLayoutOrder / kLayoutLane, or kLayoutPool
-  int waves_cap = 8;   // resident waves per compute unit a launch aims for
+  uint32_t bounds[5] = {10 * 1024, 14 * 1024, 20 * 1024, 28 * 1024, 48 * 1024};  // class bounds (bytes of row state, fam_size)
+  int layout = 0;      // index into kLayoutOrder / kLayoutLane
+  int waves_cap = 8;   // resident families per compute unit a launch aims for
 };
 // Class launch orders (largest first within a stream) and the stream of each
 // class, for the candidate layouts.  Layout 0 was chosen by hand among a
@@ -98,9 +94,8 @@ constexpr int kLayoutLane[kLayouts][6] = {  // stream of class 0..5
 // family tickets: one per class and direction, two for the FP64 pass after an
 // FP32 pass, two for the families routed to FP64 from the start, two for the
 // families whose stages do not fit LDS
-constexpr int kTickets = 19;
+constexpr int kTickets = 18;
 constexpr int kTicketHbm = 16;
-constexpr int kTicketPool = 18;  // the pooled launch
 int assign_classes(whale_batch* b);
 int plan_batch_launches(whale_batch* b);
 int ensure_gws(whale_batch* b, bool* moved);
@@ -108,9 +103,18 @@ void drop_graphs(whale_batch* b);
 uint64_t full_bytes(const whale_batch* b);
 int replan(whale_batch* b);
 
-// LDS one wave needs for family d in `mode` (fam_lds_bytes)
-size_t fam_lds(const whale::FamDev& d, int mode, bool fwd, bool root_recs) {
-  return whale::fam_lds_bytes(d, mode == WHALE_FP32_SCALED ? 4 : 8, mode != WHALE_FP64_PLAIN, fwd, root_recs);
+// LDS family d needs in `mode` when `team` waves evaluate it (fam_lds_bytes)
+size_t fam_lds(const whale::FamDev& d, int mode, bool fwd, int team, bool staged) {
+  return whale::fam_lds_bytes(d, mode == WHALE_FP32_SCALED ? 4 : 8, mode != WHALE_FP64_PLAIN, fwd, team, staged);
+}
+// The size a family is classed by: the registers its largest stage takes, at
+// 80 bytes of row state a slot (an FP32 lane's).
+size_t fam_size(const whale::FamDev& d) { return 80 * (size_t)d.max_slots; }
+// the fewest waves that hold every stage of a family in registers (kRegChunks
+// chunks a wave), at most kMaxTeam
+int fam_team(uint32_t max_slots) {
+  constexpr uint32_t held = whale::kRegChunks * whale::kChunk;
+  return std::max(1, std::min(whale::kMaxTeam, (int)((max_slots + held - 1) / held)));
 }
 }  // namespace
 
@@ -134,7 +138,7 @@ struct whale_ctx {
 struct whale_model {
   whale_ctx* ctx = nullptr;
   ModelHost h;
-  DBuf nodes, eps, phi, psi, drow, dnode, par, hlv, hnd, dlv, dnd, ebar, out;
+  DBuf nodes, eps, phi, psi, pack64, pack32, dnode, par, hlv, hnd, dlv, dnd, ebar, out;
   int n_hlevels = 0, n_dlevels = 0;
   bool has_params = false;
   std::vector<double> host_par;
@@ -145,6 +149,9 @@ struct whale_model {
     M.phi = phi.as<double>();
     M.psi = psi.as<double>();
     M.par = par.as<double>();
+    M.pack64 = pack64.as<double>();
+    M.pack32 = pack32.as<float>();
+    M.dnode = dnode.as<double>();
     M.n = h.n;
     M.n_wgd = h.n_wgd;
     M.root = h.root;
@@ -161,12 +168,12 @@ struct whale_batch {
   whale_model* model = nullptr;
   int device = 0;
   PlanHost plan;
-  DBuf fam, stage, seg, it_seg, it_gid, it_rec, it_cf, it_cg, it_bar, rec_ops, rec_sid, rec_own,
-      rec_p, clade_size, split_p, lvl, order;
-  // workspace.  ell/coef/ibar hold the main pass (FP32 or FP64 values) in
+  DBuf fam, stage, seg, run, it_gid, fs4, fs2, bs4, bs2, rec_ops, rec_p, ent_ops, ent_p, clade_size, split_p, lvl_f,
+      lvl_b, order;
+  // workspace.  ell/ibar hold the main pass (FP32 or FP64 values) in
   // their first 8 bytes per element and, for FP32 runs, the FP64 recomputation
   // of families that left the FP32 range after the first align8(4 * n) bytes.
-  DBuf ell, coef, E, ibar, fam_ll, acc, ticket, flag, fb;
+  DBuf ell, E, Eit, ibar, fam_ll, acc, ticket, flag, fb;
   // the families' split lists (per absolute clade: first split; per split:
   // g1 | g2 << 16) and, built on the first backtracking call, each
   // (family, node)'s segment and each segment's first item; the sampler's
@@ -195,7 +202,7 @@ struct whale_batch {
   // streams, and the most waves per compute unit a launch plans for.
   Tuning tune;
   // Memory budget for the stored rows of ℓ (0: none).  When the whole
-  // batch's ℓ, ī and coefficients exceed it, evaluations without stored ℓ
+  // batch's ℓ, ī and exponents exceed it, evaluations without stored ℓ
   // for the caller run the fused forward + reverse launches, whose per-wave
   // slots hold one family at a time (k_fused); their launch shapes and slots,
   // per mode, are planned on first use.
@@ -205,11 +212,10 @@ struct whale_batch {
   FusedSlots fslot[3][kClasses], fslot_hbm[3], fslot_route[3], fslot_fb[3];
   size_t fused_bytes[3] = {};
   DBuf fslots;
-  bool full_ok = false;  // ell, coef and ibar allocated for every family
-  // Deterministic gradients: reverse sweeps run one family per workgroup with
-  // the tables and accumulators in LDS, each family's accumulators land in its
-  // own slot of acc_fam, and a fixed-order sum over families follows, so that
-  // repeated evaluations give bit-identical gradients.
+  bool full_ok = false;  // ell, Eit and ibar allocated for every family
+  // Deterministic gradients: each family's accumulators land in its own slot
+  // of acc_fam, and a fixed-order sum over families follows, so that repeated
+  // evaluations give bit-identical gradients.
   bool det = false;
   DBuf acc_fam;
   // Per-family weights of the reverse sweep (whale_batch_set_seeds): n_fam
@@ -220,16 +226,12 @@ struct whale_batch {
   // the per-launch component tables, the log priors, the result and the
   // responsibilities.
   struct MixWork {
-    DBuf ell, coef, E, ibar, fam_ll, acc, ticket, flag, fb, seed, out;
+    DBuf ell, E, Eit, ibar, fam_ll, acc, ticket, flag, fb, seed, out;
   };
   std::vector<std::unique_ptr<MixWork>> mixw;
   DBuf mixsel, mixprior, mixout, mixresp;
   LaunchCfg cfg[3][2][kClasses];   // [mode][forward, backward][class]
   LaunchCfg cfg_fb[2];             // FP64 pass over families the FP32 form could not represent
-  // the pooled launch per mode (layout kLayoutPool): 0 not planned, 1 planned
-  // (pool_cfg), 2 some family of order[hbm_hi .. route_lo) does not fit the pool
-  int pool_state[3] = {};
-  LaunchCfg pool_cfg[3];
   int last_mode = -1;
   int last_launch = WHALE_LAUNCH_BATCHED;
   bool last_store_all = false;
@@ -257,19 +259,20 @@ struct whale_batch {
     B.fam = fam.as<FamDev>();
     B.stage = stage.as<StageDev>();
     B.seg = seg.as<SegDev>();
-    B.it_seg = it_seg.as<uint32_t>();
-    B.it_gid = it_gid.as<uint32_t>();
-    B.it_rec = it_rec.as<uint32_t>();
-    B.it_cf = it_cf.as<int32_t>();
-    B.it_cg = it_cg.as<int32_t>();
-    B.it_bar = it_bar.as<int32_t>();
+    B.run = run.as<SegRun>();
+    B.fs4 = fs4.as<uint32_t>();
+    B.fs2 = fs2.as<uint32_t>();
+    B.bs4 = bs4.as<uint32_t>();
+    B.bs2 = bs2.as<uint32_t>();
     B.rec_ops = rec_ops.as<uint32_t>();
-    B.rec_sid = rec_sid.as<uint32_t>();
-    B.rec_own = rec_own.as<uint16_t>();
     B.rec_p = rec_p.as<double>();
+    B.ent_ops = ent_ops.as<uint32_t>();
+    B.ent_p = ent_p.as<double>();
+    B.it_gid = it_gid.as<uint32_t>();
     B.clade_size = clade_size.as<uint16_t>();
     B.split_p = split_p.as<double>();
-    B.lvl = lvl.as<uint32_t>();
+    B.lvl_f = lvl_f.as<uint32_t>();
+    B.lvl_b = lvl_b.as<uint32_t>();
     B.order = order.as<uint32_t>();
     B.n_fam = n_fam;
     return B;
@@ -277,8 +280,8 @@ struct whale_batch {
   WorkRaw work() const {
     WorkRaw W;
     W.ell = ell.p;
-    W.coef = coef.p;
     W.E = E.as<int32_t>();
+    W.Eit = Eit.as<int32_t>();
     W.ibar = ibar.p;
     W.fam_ll = fam_ll.as<double>();
     W.acc = acc.as<double>();
@@ -292,7 +295,6 @@ struct whale_batch {
   WorkRaw work_fallback() const { return fallback_of(work()); }
   WorkRaw fallback_of(WorkRaw W) const {
     W.ell = (char*)W.ell + fp32_bytes(plan.ell_cells);
-    W.coef = (char*)W.coef + fp32_bytes(n_rec);
     W.ibar = (char*)W.ibar + fp32_bytes(plan.ibar_cells);
     return W;
   }
@@ -500,10 +502,11 @@ int whale_model_create(whale_ctx* ctx, int32_t n, const int32_t* parent, const i
   HIPCHK(m->eps.alloc(sizeof(double) * h.tab_rows));
   HIPCHK(m->phi.alloc(sizeof(double) * h.tab_rows));
   HIPCHK(m->psi.alloc(sizeof(double) * h.tab_rows));
-  HIPCHK(m->drow.alloc(sizeof(double) * 9 * h.tab_rows));
-  HIPCHK(m->dnode.alloc(sizeof(double) * 4 * n));
+  HIPCHK(m->pack64.alloc(sizeof(double) * 7 * h.tab_rows));
+  HIPCHK(m->pack32.alloc(sizeof(float) * 7 * h.tab_rows));
+  HIPCHK(m->dnode.alloc(sizeof(double) * kDnode * n));
   HIPCHK(m->par.alloc(sizeof(double) * (3 * n + nwgd + 1)));
-  HIPCHK(m->ebar.alloc(sizeof(double) * 7 * n));  // ε̄ per node, then the tail's 6 coefficients per node
+  HIPCHK(m->ebar.alloc(sizeof(double) * n));
   HIPCHK(m->out.alloc(sizeof(double) * (2 + 2 * n + nwgd)));
   *out = m.release();
   return WHALE_OK;
@@ -535,7 +538,7 @@ int whale_model_set_params(whale_model* m, const double* lambda, const double* m
   if (c->timing) HIPCHK(hipEventRecord(c->ev[0], c->stream));
   HIPCHK(hipMemcpyAsync(m->par.p, hp.data(), hp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIPCHK(launch_tables(c->stream, m->dev(), m->eps.as<double>(), m->phi.as<double>(), m->psi.as<double>(),
-                       m->drow.as<double>(), m->dnode.as<double>(), m->hlv.as<int32_t>(), m->hnd.as<int32_t>(),
+                       m->pack64.as<double>(), m->pack32.as<float>(), m->dnode.as<double>(), m->hlv.as<int32_t>(), m->hnd.as<int32_t>(),
                        m->n_hlevels));
   if (c->timing) HIPCHK(hipEventRecord(c->ev[1], c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -659,8 +662,6 @@ int whale_batch_create(whale_model* m, int32_t n_fam, const int64_t* fam_clade_o
                                (int)std::min(hw, 16u));
   if (!err.empty()) return fail(WHALE_EINVAL, err);
   PlanHost& P = b->plan;
-  if (P.rec_ops.size() > 0xffffffffull || P.it_seg.size() > 0xffffffffull)
-    return fail(WHALE_EINVAL, "batch too large");
   b->n_fam = (uint32_t)n_fam;
   b->routed.assign(n_fam, 0);
   {
@@ -677,19 +678,20 @@ int whale_batch_create(whale_model* m, int32_t n_fam, const int64_t* fam_clade_o
   HIPCHK(upload(b->fam, P.fam, st));
   HIPCHK(upload(b->stage, P.stage, st));
   HIPCHK(upload(b->seg, P.seg, st));
-  HIPCHK(upload(b->it_seg, P.it_seg, st));
+  HIPCHK(upload(b->run, P.run, st));
   HIPCHK(upload(b->it_gid, P.it_gid, st));
-  HIPCHK(upload(b->it_rec, P.it_rec, st));
-  HIPCHK(upload(b->it_cf, P.it_cf, st));
-  HIPCHK(upload(b->it_cg, P.it_cg, st));
-  HIPCHK(upload(b->it_bar, P.it_bar, st));
+  HIPCHK(upload(b->fs4, P.fs4, st));
+  HIPCHK(upload(b->fs2, P.fs2, st));
+  HIPCHK(upload(b->bs4, P.bs4, st));
+  HIPCHK(upload(b->bs2, P.bs2, st));
   HIPCHK(upload(b->rec_ops, P.rec_ops, st));
-  HIPCHK(upload(b->rec_sid, P.rec_sid, st));
-  HIPCHK(upload(b->rec_own, P.rec_own, st));
   HIPCHK(upload(b->rec_p, P.rec_p, st));
+  HIPCHK(upload(b->ent_ops, P.ent_ops, st));
+  HIPCHK(upload(b->ent_p, P.ent_p, st));
   HIPCHK(upload(b->clade_size, P.clade_size, st));
   HIPCHK(upload(b->split_p, P.split_p, st));
-  HIPCHK(upload(b->lvl, P.lvl, st));
+  HIPCHK(upload(b->lvl_f, P.lvl_f, st));
+  HIPCHK(upload(b->lvl_b, P.lvl_b, st));
   HIPCHK(upload(b->order, b->order_host, st));
   {
     std::vector<uint32_t> so(nc + 1), sg((size_t)split_off[nc]);
@@ -705,20 +707,15 @@ int whale_batch_create(whale_model* m, int32_t n_fam, const int64_t* fam_clade_o
   HIPCHK(b->flag.alloc(sizeof(uint32_t) * n_fam));
   HIPCHK(b->fb.alloc(sizeof(uint32_t) * (n_fam + 1)));
   HIPCHK(b->fam_ll.alloc(sizeof(double) * n_fam));
-  AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
+  AccLayout AL(m->h.n, m->h.n_wgd);
   HIPCHK(b->acc.alloc(sizeof(double) * AL.n));
   HIPCHK(b->ticket.alloc(sizeof(uint32_t) * kTickets));
   HIPCHK(hipHostMalloc((void**)&b->pin_out, sizeof(double) * (3 + 2 * m->h.n + m->h.n_wgd), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void**)&b->pin_fam, sizeof(double) * n_fam, hipHostMallocDefault));
   // release host copies the device now owns (keep what ℓ download needs)
-  std::vector<uint32_t>().swap(P.it_rec);
-  std::vector<int32_t>().swap(P.it_cf);
-  std::vector<int32_t>().swap(P.it_cg);
-  std::vector<int32_t>().swap(P.it_bar);
-  std::vector<uint32_t>().swap(P.rec_ops);
-  std::vector<uint32_t>().swap(P.rec_sid);
-  std::vector<uint16_t>().swap(P.rec_own);
+  for (auto* v : {&P.fs4, &P.fs2, &P.bs4, &P.bs2, &P.rec_ops, &P.ent_ops}) std::vector<uint32_t>().swap(*v);
   std::vector<double>().swap(P.rec_p);
+  std::vector<double>().swap(P.ent_p);
   *out = b.release();
   return WHALE_OK;
 }
@@ -746,7 +743,7 @@ int whale_batch_launches(const whale_batch* b, int32_t mode, int64_t* o) {
       int64_t* r = o + 8 * (whale_batch::kClasses * dir + k);
       r[0] = b->cls_hi[k] - b->cls_lo[k];
       r[1] = C.fpw;
-      r[2] = C.tabl ? 1 : 0;
+      r[2] = 0;  // the slice tables are read from global memory
       r[3] = C.grid;
       r[4] = (int64_t)C.lds();
       r[5] = C.L.shared_bytes;
@@ -785,7 +782,7 @@ int whale_batch_set_ell_budget(whale_batch* b, int64_t bytes) {
   if (b->ell_budget && full_bytes(b) > b->ell_budget && b->full_ok) {
     // the stored form's buffers are given back; a call that keeps ℓ allocates them again
     b->ell.free();
-    b->coef.free();
+    b->Eit.free();
     b->ibar.free();
     b->full_ok = false;
     if (b->last_store_all) b->last_mode = -1;  // nothing stored any more
@@ -814,7 +811,7 @@ int whale_batch_ell_bytes(const whale_batch* b, int64_t* out3) {
   for (int m = 0; m < 3; ++m)
     if (b->fused_ok[m]) fz = std::max(fz, b->fused_bytes[m]);
   out3[1] = (int64_t)fz;
-  out3[2] = (int64_t)((b->full_ok ? b->ell.n + b->coef.n + b->ibar.n : 0) + b->fslots.n);
+  out3[2] = (int64_t)((b->full_ok ? b->ell.n + b->Eit.n + b->ibar.n : 0) + b->fslots.n);
   return WHALE_OK;
 }
 
@@ -838,84 +835,79 @@ int whale_batch_stats(const whale_batch* b, int64_t* o) {
 
 namespace {
 
-// Launch shape of one forward or backward launch over families whose stages
-// hold at most `cap` items and `rcap` records.  The slice tables go to LDS
-// whenever they fit; then the shape with the most resident waves per compute
-// unit wins (LDS-limited, at most kWavesPerCU).
-constexpr int kWavesPerCU = 8;
+// Launch shape of one forward or backward launch over families that need
+// `wave` bytes of LDS each and `team` waves: the shape with the most resident
+// families per compute unit (LDS-limited, at most `cap`), then the fewest
+// families per workgroup.
 constexpr int kMaxFPW = 8;
 
-bool plan_launch(const whale_model* m, bool fwd, int mode, size_t wave, uint64_t nfam, bool multi, LaunchCfg* out,
-                 int waves_cap = kWavesPerCU) {
+bool plan_launch(const whale_model* m, bool fwd, int mode, size_t wave, uint64_t nfam, bool multi, int team,
+                 LaunchCfg* out, int cap) {
   wave = align16(std::max<size_t>(wave, 16));
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
-  auto shared_of = [&](bool tabl) {
-    return fwd ? fwd_shared_bytes(mode, tabl, m->h.tab_rows, m->h.n, m->h.n_wgd)
-               : bwd_shared_bytes(mode, tabl, m->h.tab_rows, AL.n, m->h.n, m->h.n_wgd);
-  };
-  // tables in LDS whenever some shape allows it; then the most resident waves,
-  // then the fewest families per workgroup
-  int best_fpw = 0, best_waves = 0, best_wg = 0;
-  bool best_tabl = false;
-  for (int t = 1; t >= 0 && best_fpw == 0; --t) {
-    const bool tabl = t == 1;
-    for (int fpw = 1; fpw <= (multi ? kMaxFPW : 1); ++fpw) {
-      const size_t lds = shared_of(tabl) + (size_t)fpw * wave;
-      if (lds > m->ctx->lds_wg) break;
-      const int wg = (int)std::min<size_t>(m->ctx->lds_cu / lds, (size_t)(waves_cap / fpw));
-      if (wg * fpw > best_waves) {
-        best_fpw = fpw;
-        best_waves = wg * fpw;
-        best_wg = wg;
-        best_tabl = tabl;
-      }
+  const size_t shared = fwd ? fwd_shared_bytes(mode, m->h.n, m->h.n_wgd) : bwd_shared_bytes(mode, m->h.n, m->h.n_wgd);
+  int best_fpw = 0, best_fams = 0, best_wg = 0;
+  for (int fpw = 1; fpw <= (multi && team == 1 ? kMaxFPW : 1); ++fpw) {
+    const size_t lds = shared + (size_t)fpw * wave;
+    if (lds > m->ctx->lds_wg) break;
+    const int wg = (int)std::min<size_t>(m->ctx->lds_cu / lds, (size_t)std::max(1, cap / fpw));
+    if (wg * fpw > best_fams) {
+      best_fpw = fpw;
+      best_fams = wg * fpw;
+      best_wg = wg;
     }
   }
   if (best_fpw == 0) return false;
   LaunchCfg C;
   C.fpw = best_fpw;
-  C.tabl = best_tabl;
-  C.waves_per_cu = best_waves;
+  C.team = team;
+  C.waves_per_cu = best_fams;
   C.L.wave_bytes = (uint32_t)wave;
-  C.L.shared_bytes = (uint32_t)shared_of(C.tabl);
+  C.L.shared_bytes = (uint32_t)shared;
   const uint64_t need = (nfam + C.fpw - 1) / C.fpw;
   C.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)m->ctx->n_cu * best_wg, need));
   *out = C;
   return true;
 }
 
-// a launch over the families `fams`: the wave region fits the largest of
-// them, with the root records staged in LDS unless reading them from global
-// memory lets more waves share a compute unit
+// A launch over the families `fams` (both directions when `fused`): a
+// family's region fits the largest of them, its team the widest stage.
 bool plan_families(const whale_batch* b, bool fwd, int mode, const uint32_t* fams, size_t nf, uint64_t grid_fams,
-                   bool multi, LaunchCfg* out, bool force_gws = false) {
-  size_t with = 16, without = 16;
-  for (size_t j = 0; j < nf; ++j) {
-    const FamDev& d = b->plan.fam[fams[j]];
-    with = std::max(with, fam_lds(d, mode, fwd, true));
-    without = std::max(without, fam_lds(d, mode, fwd, false));
+                   bool multi, LaunchCfg* out, bool force_gws = false, bool fused = false) {
+  uint32_t slots = 0;
+  for (size_t j = 0; j < nf; ++j) slots = std::max(slots, b->plan.fam[fams[j]].max_slots);
+  auto need_of = [&](int team, bool staged) {
+    size_t need = 16;
+    for (size_t j = 0; j < nf; ++j) {
+      const FamDev& d = b->plan.fam[fams[j]];
+      need = std::max(need, fam_lds(d, mode, fwd, team, staged));
+      if (fused) need = std::max(need, fam_lds(d, mode, !fwd, team, staged));
+    }
+    return need;
+  };
+  const int team = fam_team(slots);
+  // the root's terms are staged in LDS unless reading them from global memory
+  // lets more than a third more families share a compute unit
+  LaunchCfg x, y;
+  const int cap = b->tune.waves_cap;
+  const bool ox = !force_gws && plan_launch(b->model, fwd, mode, need_of(team, true), grid_fams, multi, team, &x, cap);
+  const bool oy = !force_gws && plan_launch(b->model, fwd, mode, need_of(team, false), grid_fams, multi, team, &y, cap);
+  if (ox || oy) {
+    *out = ox && (!oy || 4 * x.waves_per_cu >= 3 * y.waves_per_cu) ? x : y;
+    return true;
   }
-  LaunchCfg a, c;
-  const bool det = b->det && !fwd;  // deterministic reverse sweep: one family per workgroup, tables in LDS
-  if (det) multi = false;
-  const bool oa = !force_gws && plan_launch(b->model, fwd, mode, with, grid_fams, multi, &a, b->tune.waves_cap);
-  const bool oc = !force_gws && plan_launch(b->model, fwd, mode, without, grid_fams, multi, &c, b->tune.waves_cap);
-  if (oa && (!oc || a.waves_per_cu >= c.waves_per_cu)) *out = a;
-  else if (oc) *out = c;
-  if ((oa || oc) && (!det || out->tabl)) return true;
-  // the stage buffers in global memory: one wave per workgroup, root records
-  // read from global memory, only the node constants (and accumulators) in LDS
+  // the stage buffers in global memory: one family per workgroup by the
+  // largest team, only the node constants (and accumulators) in LDS
   const whale_model* m = b->model;
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
+  const size_t need = need_of(kMaxTeam, false);
   LaunchCfg g;
   g.gws = true;
   g.fpw = 1;
-  g.tabl = det;
+  g.team = kMaxTeam;
   g.waves_per_cu = 1;
-  g.L.wave_bytes = (uint32_t)align16(without);
-  g.L.shared_bytes = (uint32_t)(fwd ? fwd_shared_bytes(mode, false, m->h.tab_rows, m->h.n, m->h.n_wgd)
-                                    : bwd_shared_bytes(mode, det, m->h.tab_rows, AL.n, m->h.n, m->h.n_wgd));
-  if (g.L.shared_bytes > m->ctx->lds_wg || without > 0xffffffffull) return false;
+  g.L.wave_bytes = (uint32_t)align16(need);
+  g.L.shared_bytes = (uint32_t)(fwd ? fwd_shared_bytes(mode, m->h.n, m->h.n_wgd)
+                                    : bwd_shared_bytes(mode, m->h.n, m->h.n_wgd));
+  if (g.L.shared_bytes > m->ctx->lds_wg || need > 0xffffffffull) return false;
   g.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)m->ctx->n_cu, grid_fams));
   *out = g;
   return true;
@@ -925,14 +917,12 @@ bool plan_families(const whale_batch* b, bool fwd, int mode, const uint32_t* fam
 // stages (the largest form) fit the LDS limit in both directions
 bool fits_lds(const whale_batch* b, const FamDev& d) {
   const whale_model* m = b->model;
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
   size_t lim = m->ctx->lds_wg;
   if (b->lds_limit) lim = std::min(lim, b->lds_limit);
-  const int md = WHALE_FP64_SCALED;
-  const size_t f = fwd_shared_bytes(md, false, m->h.tab_rows, m->h.n, m->h.n_wgd) +
-                   align16(std::max<size_t>(16, fam_lds(d, md, true, false)));
-  const size_t r = bwd_shared_bytes(md, false, m->h.tab_rows, AL.n, m->h.n, m->h.n_wgd) +
-                   align16(std::max<size_t>(16, fam_lds(d, md, false, false)));
+  const int md = WHALE_FP64_SCALED, team = fam_team(d.max_slots);
+  const size_t f = fwd_shared_bytes(md, m->h.n, m->h.n_wgd) + align16(fam_lds(d, md, true, team, false));
+  const size_t r =
+      bwd_shared_bytes(md, m->h.n, m->h.n_wgd) + align16(fam_lds(d, md, false, team, false));
   return f <= lim && r <= lim;
 }
 
@@ -960,8 +950,8 @@ int plan_batch_launches(whale_batch* b) {
   return WHALE_OK;
 }
 
-// Size classes by the LDS one family needs (FP32, either direction), so that
-// each launch packs as many families per compute unit as their LDS allows.
+// Size classes by the widest stage of a family (fam_size), so that the
+// families of a launch want the same number of waves.
 // Order: largest class first, costliest families first in a class, families
 // routed to FP64 last.  Then the launch shapes.
 int assign_classes(whale_batch* b) {
@@ -977,8 +967,7 @@ int assign_classes(whale_batch* b) {
       hbm.push_back(f);
       continue;
     }
-    const size_t need = std::max(fam_lds(P.fam[f], WHALE_FP32_SCALED, true, true),
-                                 fam_lds(P.fam[f], WHALE_FP32_SCALED, false, true));
+    const size_t need = fam_size(P.fam[f]);
     int k = whale_batch::kClasses - 1;
     while (k > 0 && need <= bounds[k - 1]) --k;
     cls[k].push_back(f);
@@ -995,7 +984,6 @@ int assign_classes(whale_batch* b) {
   b->route_lo = (uint32_t)b->order_host.size();
   b->order_host.insert(b->order_host.end(), rt.begin(), rt.end());
   for (bool& x : b->fused_ok) x = false;  // fused shapes follow the classes
-  for (int& x : b->pool_state) x = 0;     // so does the pooled launch's family range
   int rc = plan_batch_launches(b);
   if (rc != WHALE_OK) return rc;
   for (int mode = 0; mode < 3; ++mode)
@@ -1026,7 +1014,7 @@ int ensure_gws(whale_batch* b, bool* moved) {
     }
   for (uint32_t k = b->hbm_lo; k < b->hbm_hi; ++k)
     for (int dir = 0; dir < 2; ++dir)
-      main = std::max(main, align16(fam_lds(b->plan.fam[b->order_host[k]], WHALE_FP64_SCALED, dir == 0, false)));
+      main = std::max(main, align16(fam_lds(b->plan.fam[b->order_host[k]], WHALE_FP64_SCALED, dir == 0, kMaxTeam, false)));
   main = (main + 255) & ~(size_t)255;
   const size_t need = main + route;
   if (moved) *moved = main != b->gws_main || need > b->gws.n;
@@ -1047,11 +1035,11 @@ void drop_graphs(whale_batch* b) {
           }
 }
 
-// ℓ, coefficients and ī of every family (8 bytes per value, or 4 with the
-// FP64 region of recomputed families after it in the FP32 form)
+// ℓ and ī of every family (8 bytes per value, or 4 with the FP64 region of
+// recomputed families after it in the FP32 form) and the items' exponents
 uint64_t full_bytes(const whale_batch* b) {
   const PlanHost& P = b->plan;
-  return (16 + 12 * std::max<uint64_t>(1, P.ell_cells)) + (16 + 12 * std::max<uint64_t>(1, b->n_rec)) +
+  return (16 + 12 * std::max<uint64_t>(1, P.ell_cells)) + 4 * std::max<uint64_t>(1, P.it_seg.size()) +
          (16 + 12 * std::max<uint64_t>(1, P.ibar_cells));
 }
 
@@ -1059,62 +1047,30 @@ int ensure_full(whale_batch* b) {
   if (b->full_ok) return WHALE_OK;
   const PlanHost& P = b->plan;
   HIPCHK(b->ell.alloc(16 + 12 * std::max<uint64_t>(1, P.ell_cells)));
-  HIPCHK(b->coef.alloc(16 + 12 * std::max<uint64_t>(1, b->n_rec)));
+  HIPCHK(b->Eit.alloc(4 * std::max<uint64_t>(1, P.it_seg.size())));
   HIPCHK(b->ibar.alloc(16 + 12 * std::max<uint64_t>(1, P.ibar_cells)));
   b->full_ok = true;
   return WHALE_OK;
 }
 
-// launch shape of a fused launch over `fams`: the wave's stage region fits
-// both directions, the shared LDS is the reverse sweep's
-bool plan_fused_launch(const whale_batch* b, int mode, const uint32_t* fams, size_t nf, uint64_t grid_fams, bool multi,
-                       bool force_gws, LaunchCfg* out) {
-  size_t with = 16, without = 16;
-  for (size_t j = 0; j < nf; ++j) {
-    const FamDev& d = b->plan.fam[fams[j]];
-    with = std::max({with, fam_lds(d, mode, true, true), fam_lds(d, mode, false, true)});
-    without = std::max({without, fam_lds(d, mode, true, false), fam_lds(d, mode, false, false)});
-  }
-  const whale_model* m = b->model;
-  LaunchCfg a, c;
-  if (b->det) multi = false;
-  const bool oa = !force_gws && plan_launch(m, false, mode, with, grid_fams, multi, &a, b->tune.waves_cap);
-  const bool oc = !force_gws && plan_launch(m, false, mode, without, grid_fams, multi, &c, b->tune.waves_cap);
-  if (oa && (!oc || a.waves_per_cu >= c.waves_per_cu)) *out = a;
-  else if (oc) *out = c;
-  if ((oa || oc) && (!b->det || out->tabl)) return true;
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
-  LaunchCfg g;
-  g.gws = true;
-  g.fpw = 1;
-  g.tabl = false;  // the fused kernel's global-memory form keeps the tables in global memory
-  g.waves_per_cu = 1;
-  g.L.wave_bytes = (uint32_t)align16(without);
-  g.L.shared_bytes = (uint32_t)bwd_shared_bytes(mode, false, m->h.tab_rows, AL.n, m->h.n, m->h.n_wgd);
-  if (g.L.shared_bytes > m->ctx->lds_wg || without > 0xffffffffull) return false;
-  g.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)m->ctx->n_cu, grid_fams));
-  *out = g;
-  return true;
-}
-
-// a slot of a fused launch over `fams`: the largest family's rows, ī and coefficients
+// a slot of a fused launch over `fams`: the largest family's rows, ī and exponents
 void fused_slot(const whale_batch* b, int mode, const uint32_t* fams, size_t nf, FusedSlots* out) {
   const PlanHost& P = b->plan;
   const uint64_t s = mode == WHALE_FP32_SCALED ? 4 : 8;
-  uint64_t cells = 1, ibar = 1, recs = 1;
+  uint64_t cells = 1, ibar = 1, items = 1;
   for (size_t j = 0; j < nf; ++j) {
     const uint32_t f = fams[j];
     const FamDev& d = P.fam[f];
     const bool last = f + 1 == b->n_fam;
     cells = std::max(cells, (last ? P.ell_cells : P.fam[f + 1].ell0) - d.ell0);
     ibar = std::max(ibar, (last ? P.ibar_cells : P.fam[f + 1].ibar0) - d.ibar0);
-    recs = std::max<uint64_t>(recs, d.n_recs);
+    items = std::max<uint64_t>(items, d.n_items);
   }
   auto al = [](uint64_t x) { return (x + 255) & ~(uint64_t)255; };
   FusedSlots S;
   S.ibar_off = al(cells * s);
-  S.coef_off = S.ibar_off + al(ibar * s);
-  S.slot_bytes = S.coef_off + al(recs * s);
+  S.eit_off = S.ibar_off + al(ibar * s);
+  S.slot_bytes = S.eit_off + al(items * 4);
   *out = S;
 }
 
@@ -1131,27 +1087,27 @@ int plan_fused(whale_batch* b, int mode) {
   for (int k = 0; k < whale_batch::kClasses; ++k) {
     const uint32_t lo = b->cls_lo[k], hi = b->cls_hi[k];
     if (hi == lo) continue;
-    if (!plan_fused_launch(b, mode, ord + lo, hi - lo, hi - lo, true, false, &b->fcfg[mode][k]))
+    if (!plan_families(b, false, mode, ord + lo, hi - lo, hi - lo, true, &b->fcfg[mode][k], false, true))
       return fail(WHALE_EINVAL, "no fused launch shape");
     fused_slot(b, mode, ord + lo, hi - lo, &b->fslot[mode][k]);
     items.push_back({&b->fcfg[mode][k], &b->fslot[mode][k]});
   }
   if (b->hbm_hi > b->hbm_lo) {
     const uint32_t nh = b->hbm_hi - b->hbm_lo;
-    if (!plan_fused_launch(b, mode, ord + b->hbm_lo, nh, nh, false, true, &b->fcfg_hbm[mode]))
+    if (!plan_families(b, false, mode, ord + b->hbm_lo, nh, nh, false, &b->fcfg_hbm[mode], true, true))
       return fail(WHALE_EINVAL, "no fused launch shape");
     fused_slot(b, mode, ord + b->hbm_lo, nh, &b->fslot_hbm[mode]);
     items.push_back({&b->fcfg_hbm[mode], &b->fslot_hbm[mode]});
   }
   if (b->route_lo < b->n_fam) {
     const uint32_t nr = b->n_fam - b->route_lo;
-    if (!plan_fused_launch(b, smode, ord + b->route_lo, nr, nr, true, false, &b->fcfg_route[mode]))
+    if (!plan_families(b, false, smode, ord + b->route_lo, nr, nr, true, &b->fcfg_route[mode], false, true))
       return fail(WHALE_EINVAL, "no fused launch shape");
     fused_slot(b, smode, ord + b->route_lo, nr, &b->fslot_route[mode]);
     items.push_back({&b->fcfg_route[mode], &b->fslot_route[mode]});
   }
   if (mode == WHALE_FP32_SCALED) {
-    if (!plan_fused_launch(b, WHALE_FP64_SCALED, ord, b->n_fam, (uint64_t)m->ctx->n_cu, false, false, &b->fcfg_fb))
+    if (!plan_families(b, false, WHALE_FP64_SCALED, ord, b->n_fam, (uint64_t)m->ctx->n_cu, false, &b->fcfg_fb, false, true))
       return fail(WHALE_EINVAL, "no fused launch shape");
     fused_slot(b, WHALE_FP64_SCALED, ord, b->n_fam, &b->fslot_fb[mode]);
     items.push_back({&b->fcfg_fb, &b->fslot_fb[mode]});
@@ -1185,40 +1141,6 @@ int plan_fused(whale_batch* b, int mode) {
   return WHALE_OK;
 }
 
-// the class layout the class launches use (layout 0 when the pooled layout is
-// chosen but a call cannot use it)
-int class_layout(const whale_batch* b) { return b->tune.layout < kLayouts ? b->tune.layout : 0; }
-
-// The pooled launch of `mode`: one workgroup per compute unit holding its
-// LDS, the reverse sweep's shared area (tables in LDS), the rest a pool of
-// pages.  False when the shared area leaves no pool or some family of
-// order[hbm_hi .. route_lo) does not fit it.
-bool pool_ok(whale_batch* b, int mode) {
-  int& st = b->pool_state[mode];
-  if (st) return st == 1;
-  st = 2;
-  const whale_model* m = b->model;
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
-  const size_t shared = bwd_shared_bytes(mode, true, m->h.tab_rows, AL.n, m->h.n, m->h.n_wgd);
-  const size_t lim = m->ctx->lds_wg;  // (an LDS limit only moves families to the global-memory path)
-  if (shared + kPoolHdrBytes + kPage > lim) return false;
-  const size_t pages = std::min<size_t>((lim - shared - kPoolHdrBytes) / kPage, (kPoolHdrBytes / 4 - 1) * 32);
-  const size_t pool = pages * kPage;
-  const size_t s = mode == WHALE_FP32_SCALED ? 4 : 8;
-  for (uint32_t k = b->hbm_hi; k < b->route_lo; ++k)
-    if (pool_need(b->plan.fam[b->order_host[k]], s, mode != WHALE_FP64_PLAIN, pool) > pool) return false;
-  LaunchCfg C;
-  C.grid = std::max(1, std::min<int>(m->ctx->n_cu, (int)(b->route_lo - b->hbm_hi)));
-  C.fpw = kPoolWaves;
-  C.tabl = true;
-  C.waves_per_cu = kPoolWaves;
-  C.L.shared_bytes = (uint32_t)shared;
-  C.L.wave_bytes = (uint32_t)(kPoolHdrBytes + pool);
-  b->pool_cfg[mode] = C;
-  st = 1;
-  return true;
-}
-
 bool use_fused(const whale_batch* b, int32_t launch, bool keep) {
   return b->ell_budget && launch == WHALE_LAUNCH_BATCHED && !keep && full_bytes(b) > b->ell_budget;
 }
@@ -1237,7 +1159,7 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   WorkRaw W = ws ? *ws : b->work();
   W.acc_fam = b->det && grad ? b->acc_fam.as<double>() : nullptr;
   W.seed = b->seeded && grad ? b->seed.as<double>() : nullptr;
-  const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
+  const AccLayout AL(m->h.n, m->h.n_wgd);
   if (timed) HIPCHK(hipEventRecord(c->ev[1], st));
   HIPCHK(launch_fill_u32(st, W.ticket, 0u, kTickets));
   if (grad) HIPCHK(launch_fill_f64(st, W.acc, 0.0, AL.n));
@@ -1259,8 +1181,8 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
     // classes in launch order and their streams
-    const int* kOrder = kLayoutOrder[class_layout(b)];
-    auto lane_of = [&](int k) { return kLayoutLane[class_layout(b)][k]; };
+    const int* kOrder = kLayoutOrder[b->tune.layout];
+    auto lane_of = [&](int k) { return kLayoutLane[b->tune.layout][k]; };
     bool used[kLanes] = {};
     for (int k = 0; k < whale_batch::kClasses; ++k)
       if (b->cls_hi[k] > b->cls_lo[k]) used[lane_of(k)] = true;
@@ -1299,8 +1221,8 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   auto interleaved = [&]() -> int {
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
-    const int* kOrder = kLayoutOrder[class_layout(b)];
-    const int* kLane = kLayoutLane[class_layout(b)];
+    const int* kOrder = kLayoutOrder[b->tune.layout];
+    const int* kLane = kLayoutLane[b->tune.layout];
     bool used[kLanes] = {};
     for (int k = 0; k < whale_batch::kClasses; ++k)
       if (b->cls_hi[k] > b->cls_lo[k]) used[kLane[k]] = true;
@@ -1367,8 +1289,8 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
     }
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
-    const int* kOrder = kLayoutOrder[class_layout(b)];
-    const int* kLane = kLayoutLane[class_layout(b)];
+    const int* kOrder = kLayoutOrder[b->tune.layout];
+    const int* kLane = kLayoutLane[b->tune.layout];
     bool used[kLanes] = {};
     for (int k = 0; k < whale_batch::kClasses; ++k)
       if (b->cls_hi[k] > b->cls_lo[k]) used[kLane[k]] = true;
@@ -1420,27 +1342,8 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
     HIPCHK(hipEventRecord(c->fork[7], c->side2));
   }
   // per-kernel timing keeps the forward and reverse phases apart
-  const bool pooled = launch == WHALE_LAUNCH_BATCHED && b->tune.layout == kLayoutPool && !W.acc_fam && pool_ok(b, mode);
-  const bool inter = !pooled && launch == WHALE_LAUNCH_BATCHED && grad && !timed;
-  if (pooled) {
-    // families in global memory (both directions), then one pooled launch
-    // over the others: both directions per family, so the reverse phase of
-    // per-kernel timing holds only the FP64 pass's reverse sweep
-    if (b->hbm_hi > b->hbm_lo) {
-      WorkRaw Wh = W;
-      Wh.ticket = W.ticket + kTicketHbm;
-      HIPCHK(launch_forward(mode, store_all, b->cfg_hbm[mode][0], st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
-      if (grad) {
-        Wh.ticket = W.ticket + kTicketHbm + 1;
-        HIPCHK(launch_backward(mode, b->cfg_hbm[mode][1], st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
-      }
-    }
-    if (b->route_lo > b->hbm_hi) {
-      WorkRaw Wp = W;
-      Wp.ticket = W.ticket + kTicketPool;
-      HIPCHK(launch_pool(mode, store_all, b->pool_cfg[mode], st, B, M, Wp, b->hbm_hi, b->route_lo, grad ? 1 : 0));
-    }
-  } else if (inter) {
+  const bool inter = launch == WHALE_LAUNCH_BATCHED && grad && !timed;
+  if (inter) {
     if ((rc = interleaved()) != WHALE_OK) return rc;
   } else if (launch == WHALE_LAUNCH_BATCHED) {
     if ((rc = batched(0)) != WHALE_OK) return rc;
@@ -1454,7 +1357,7 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   }
   if (timed) HIPCHK(hipEventRecord(c->ev[2], st));
   if (grad) {
-    if (inter || pooled) {
+    if (inter) {
       // the reverse sweeps ran above
     } else if (launch == WHALE_LAUNCH_BATCHED) {
       if ((rc = batched(1)) != WHALE_OK) return rc;
@@ -1473,7 +1376,7 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   }
   if (W.acc_fam) HIPCHK(launch_det_sum(st, W.acc_fam, nf, AL.n, W.acc));
   double* out = ws_out ? ws_out : m->out.as<double>();
-  HIPCHK(launch_tail(st, M, W.fam_ll, nf, W.acc, m->ebar.as<double>(), m->drow.as<double>(), m->dnode.as<double>(),
+  HIPCHK(launch_tail(st, M, W.fam_ll, nf, W.acc, m->ebar.as<double>(),
                      m->dlv.as<int32_t>(), m->dnd.as<int32_t>(), m->n_dlevels, m->h.cond, grad ? 1 : 0, out,
                      W.seed ? W.seed + nf : nullptr));
   if (timed) HIPCHK(hipEventRecord(c->ev[4], st));
@@ -1509,7 +1412,7 @@ int run(whale_batch* b, int32_t mode_in, int32_t launch, bool grad, double* out_
   }
   const bool fused = use_fused(b, launch, keep);
   if (b->det && grad) {
-    const AccLayout AL(m->h.tab_rows, m->h.n, m->h.n_wgd);
+    const AccLayout AL(m->h.n, m->h.n_wgd);
     HIPCHK(b->acc_fam.alloc(sizeof(double) * (size_t)b->n_fam * AL.n));
   }
   if (fused) {
@@ -1629,8 +1532,8 @@ void tune_key(const whale_batch* b, int mode, bool grad, std::string* key) {
   for (const FamDev& d : b->plan.fam) {
     mix(d.n_clades);
     mix(d.max_items);
-    mix(d.max_recs);
-    mix(d.root_recs);
+    mix(d.max_slots);
+    mix(d.n_recs);
     mix(d.n_stages);
   }
   hipDeviceProp_t prop;
@@ -1644,14 +1547,8 @@ void tune_key(const whale_batch* b, int mode, bool grad, std::string* key) {
   *key = buf;
 }
 
-// The pooled launch is switched off: its first GPU run ended in a memory
-// fault whose cause is not identified (the allocator and the per-family
-// LDS bounds check out on the CPU), so no tuning may select it.
-constexpr bool kPoolEnabled = false;
-
 bool valid_tuning(const Tuning& t) {
-  const int last = kPoolEnabled ? kLayoutPool : kLayouts - 1;
-  if (t.layout < 0 || t.layout > last || t.waves_cap < 1 || t.waves_cap > 32) return false;
+  if (t.layout < 0 || t.layout >= kLayouts || t.waves_cap < 1 || t.waves_cap > 32) return false;
   for (int i = 0; i < 5; ++i) {
     if (t.bounds[i] < 1024) return false;
     if (i > 0 && t.bounds[i] <= t.bounds[i - 1]) return false;
@@ -1740,7 +1637,7 @@ int whale_batch_autotune(whale_batch* b, int32_t mode, int32_t gradient, int32_t
     // fastest: their basins differ, and at the starting bounds the two are
     // often within the timing noise of each other
     std::vector<std::pair<double, int>> lay{{t_start, start.layout}};
-    for (int l = 0; l <= (kPoolEnabled ? kLayoutPool : kLayouts - 1); ++l) {
+    for (int l = 0; l < kLayouts; ++l) {
       if (l == start.layout) continue;
       Tuning t = start;
       t.layout = l;
@@ -1762,7 +1659,7 @@ int whale_batch_autotune(whale_batch* b, int32_t mode, int32_t gradient, int32_t
       for (int round = 0; round < 2; ++round) {
         const Tuning before = best;
         if (round > 0)
-          for (int l = 0; l <= (kPoolEnabled ? kLayoutPool : kLayouts - 1); ++l) {
+          for (int l = 0; l < kLayouts; ++l) {
             if (l == best.layout) continue;
             Tuning t = best;
             t.layout = l;
@@ -1843,7 +1740,7 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
   const uint32_t nf = b->n_fam;
   const bool fp32 = mode == WHALE_FP32_SCALED;
   const bool grad = gradient != 0;
-  const AccLayout AL(H.tab_rows, H.n, H.n_wgd);
+  const AccLayout AL(H.n, H.n_wgd);
   const int ng = 2 + 2 * H.n + H.n_wgd;  // a tail's output
   // workspaces, sized as the batch's own
   while ((int)b->mixw.size() < K) b->mixw.emplace_back(new whale_batch::MixWork());
@@ -1851,7 +1748,7 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
   for (int j = 0; j < K; ++j) {
     whale_batch::MixWork& x = *b->mixw[j];
     HIPCHK(x.ell.alloc(b->ell.n));
-    HIPCHK(x.coef.alloc(b->coef.n));
+    HIPCHK(x.Eit.alloc(b->Eit.n));
     HIPCHK(x.E.alloc(b->E.n));
     HIPCHK(x.ibar.alloc(b->ibar.n));
     HIPCHK(x.fam_ll.alloc(b->fam_ll.n));
@@ -1863,7 +1760,7 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
     HIPCHK(x.out.alloc(sizeof(double) * ng));
     WorkRaw W;
     W.ell = x.ell.p;
-    W.coef = x.coef.p;
+    W.Eit = x.Eit.as<int32_t>();
     W.E = x.E.as<int32_t>();
     W.ibar = x.ibar.p;
     W.fam_ll = x.fam_ll.as<double>();
@@ -1931,8 +1828,8 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
   // one direction: every size class as one launch over all components on the
   // three streams, the families routed to FP64 as one launch beside them, and
   // the FP64 pass over the families each component's FP32 pass flagged
-  const int* kOrder = kLayoutOrder[class_layout(b)];
-  const int* kLane = kLayoutLane[class_layout(b)];
+  const int* kOrder = kLayoutOrder[b->tune.layout];
+  const int* kLane = kLayoutLane[b->tune.layout];
   auto direction = [&](int dir) -> int {
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
@@ -1990,8 +1887,7 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
     if ((rc = direction(1)) != WHALE_OK) return rc;
     for (int j = 0; j < K; ++j) {
       const whale_model* m = comps[j];
-      HIPCHK(launch_tail(st, m->dev(), Wj[j].fam_ll, nf, Wj[j].acc, m->ebar.as<double>(), m->drow.as<double>(),
-                         m->dnode.as<double>(), m->dlv.as<int32_t>(), m->dnd.as<int32_t>(), m->n_dlevels, H.cond, 1,
+      HIPCHK(launch_tail(st, m->dev(), Wj[j].fam_ll, nf, Wj[j].acc, m->ebar.as<double>(), m->dlv.as<int32_t>(), m->dnd.as<int32_t>(), m->n_dlevels, H.cond, 1,
                          b->mixw[j]->out.as<double>(), Wj[j].seed + nf));
     }
   }
@@ -2053,7 +1949,7 @@ int whale_batch_set_seeds(whale_batch* b, const double* seeds) {
 int whale_batch_pooled(whale_batch* b, int32_t mode, int32_t* out) {
   if (!b || !out) return fail(WHALE_EINVAL, "NULL argument");
   if (mode < 0 || mode > 2) return fail(WHALE_EINVAL, "unknown mode");
-  *out = b->tune.layout == kLayoutPool && !b->det && pool_ok(b, mode) ? 1 : 0;
+  *out = 0;
   return WHALE_OK;
 }
 
@@ -2120,7 +2016,7 @@ int whale_logpdf_noalloc(whale_batch* b, int32_t mode, double* d_family, double*
   unsigned char* base = c->scratch;
   WorkRaw W{};
   W.ell = base + o_ell;
-  W.coef = base + o_ell;   // not read or written without stored rows
+  W.Eit = nullptr;         // not read or written without stored rows
   W.ibar = base + o_ell;   // not read or written without a gradient
   W.acc = nullptr;         // not read or written without a gradient
   W.E = reinterpret_cast<int32_t*>(base + o_E);

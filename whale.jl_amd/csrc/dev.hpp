@@ -12,19 +12,20 @@ struct BatchDev {
   const FamDev* fam;
   const StageDev* stage;
   const SegDev* seg;
-  const uint32_t* it_seg;
-  const uint32_t* it_gid;
-  const uint32_t* it_rec;
-  const int32_t* it_cf;
-  const int32_t* it_cg;
-  const int32_t* it_bar;
+  const SegRun* run;
+  const uint32_t* fs4;   // slots: 4 and 2 words each (plan.hpp)
+  const uint32_t* fs2;
+  const uint32_t* bs4;
+  const uint32_t* bs2;
   const uint32_t* rec_ops;
-  const uint32_t* rec_sid;
-  const uint16_t* rec_own;
   const double* rec_p;
+  const uint32_t* ent_ops;
+  const double* ent_p;
+  const uint32_t* it_gid;
   const uint16_t* clade_size;
   const double* split_p;
-  const uint32_t* lvl;
+  const uint32_t* lvl_f;
+  const uint32_t* lvl_b;
   const uint32_t* order;   // families in processing order
   uint32_t n_fam;
 };
@@ -35,17 +36,31 @@ struct ModelDev {
   const double* phi;
   const double* psi;
   const double* par;       // [λ(n), μ(n), p(n), q(n_wgd), η]
+  // the slice tables as the DP reads them, in FP64 and FP32: per row φ, χ = ψ/β,
+  // D_α, D_β; then per row φ, ψ; then per row D_ε0 (k_tables)
+  const double* pack64;
+  const float* pack32;
+  const double* dnode;     // per node kDnode values (k_tables)
   int n;
   int n_wgd;
   int root;
   int tab_rows;
 };
 
-// type-erased workspace (ell, coef, ibar hold float or double)
+// per node: ∂α/∂λ, ∂α/∂μ, ∂β/∂λ, ∂β/∂μ; 1/(1-α), 1/(1-β), β; ∂ε_top/∂(ε of
+// row 0), ∂ε_top/∂α, ∂ε_top/∂β (all 0 for a node of one row)
+constexpr int kDnode = 10;
+
+__device__ __forceinline__ double eps_top(const ModelDev& M, int node) {
+  const NodeDev& d = M.node[node];
+  return M.eps[d.tab + d.R - 1];
+}
+
+// type-erased workspace (ell, ibar hold float or double)
 struct WorkRaw {
   void* ell;
-  void* coef;
-  int32_t* E;
+  int32_t* E;         // per clade
+  int32_t* Eit;       // per item
   void* ibar;
   double* fam_ll;
   double* acc;
@@ -60,14 +75,17 @@ struct WorkRaw {
   double* seed = nullptr;
 };
 
-// gradient accumulator layout (doubles)
+// gradient accumulator layout (doubles): per node the derivatives of logL in
+// the branch's α, β and ε of row 0 through its φ_r, ψ_r, and in ε at its top;
+// then q per WGD and the root's constants
 struct AccLayout {
-  int phi, psi, eps, q, rootA, rootB, n;
-  __host__ __device__ AccLayout(int tab_rows, int nodes, int nwgd) {
-    phi = 0;
-    psi = tab_rows;
-    eps = 2 * tab_rows;
-    q = eps + nodes;
+  int da, db, e0, eps, q, rootA, rootB, n;
+  __host__ __device__ AccLayout(int nodes, int nwgd) {
+    da = 0;
+    db = nodes;
+    e0 = 2 * nodes;
+    eps = 3 * nodes;
+    q = 4 * nodes;
     rootA = q + nwgd;
     rootB = rootA + 1;
     n = rootB + 1;
@@ -76,87 +94,78 @@ struct AccLayout {
 
 __host__ __device__ constexpr size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
-// LDS of one wave, laid out afresh for every stage from its item count n and
-// record count nr (s = bytes per Real).  The same functions size the launches
-// on the host and carve the buffers on the device.
-//   forward stage:  bA bB bF sAcc [n] | sCoef sP [nr] | sOps [nr] | sOwn [nr] (u16) |
-//                   sRO [n+1] | sSegL [n] (u16) | sEi [n] | sFlag [n] (scaled forms)
-//   forward root:   bA bF bB [n] | sCoef [nr] | sOps [nr] | sOwn [nr] (u16) | sRO [n+1] | sEi [n] (scaled)
-//   reverse stage:  bA bB bV bG sFo [n] | sCoef [nr] | sOps [nr] | sOwn [nr] (u16) |
-//                   sRO [n+1] | sSegL [n] (u16)
-//   reverse root:   bA bB bV bG [n] | sCoef [nr] | sOps [nr] | sOwn [nr] (u16) | sRO [n+1]
-// (root records are staged only when they fit: nr = 0 reads them from global memory)
-__host__ __device__ inline size_t fwd_stage_bytes(size_t s, bool scaled, size_t n, size_t nr) {
-  return align16(4 * n * s) + align16(2 * nr * s) + align16(4 * nr) + align16(2 * nr) + align16(4 * (n + 1)) +
-         align16(2 * n) + (scaled ? align16(4 * n) + align16(n) : 0);
+// Chunks of slots a wave holds in registers; a stage with more than its team
+// holds streams the rest from memory every row.
+constexpr int kRegChunks = 1;
+constexpr int kMaxTeam = 12;  // most waves of one family (three a SIMD)
+
+// LDS of one family, laid out afresh for every stage from its item count n
+// (s = bytes per Real).  The same functions size the launches on the host and
+// carve the buffers on the device.
+//   forward stage, root:  A F G [n] | E [n], flags [n] (scaled forms)
+//   reverse stage:        five arrays [n] | row sums, 5 doubles an item, when the
+//                         stage has more slots than the largest team's registers
+//   reverse root:         A V F G [n] | E [n] (scaled forms)
+__host__ __device__ inline size_t fwd_bytes(size_t s, bool scaled, size_t n) {
+  return align16(3 * n * s) + (scaled ? align16(4 * n) + align16(n) : 0);
 }
-__host__ __device__ inline size_t fwd_root_bytes(size_t s, bool scaled, size_t n, size_t nr) {
-  return align16(3 * n * s) + align16(nr * s) + align16(4 * nr) + align16(2 * nr) + align16(4 * (n + 1)) +
-         (scaled ? align16(4 * n) : 0);
+__host__ __device__ inline size_t bwd_stage_bytes(size_t s, size_t n, size_t slots) {
+  return align16(5 * n * s) + (slots > kRegChunks * (size_t)kChunk ? 40 * n : 0);
 }
-__host__ __device__ inline size_t bwd_stage_bytes(size_t s, size_t n, size_t nr) {
-  return align16(5 * n * s) + align16(nr * s) + align16(4 * nr) + align16(2 * nr) + align16(4 * (n + 1)) +
-         align16(2 * n);
-}
-__host__ __device__ inline size_t bwd_root_bytes(size_t s, size_t n, size_t nr) {
-  return align16(4 * n * s) + align16(nr * s) + align16(4 * nr) + align16(2 * nr) + align16(4 * (n + 1));
+__host__ __device__ inline size_t bwd_root_bytes(size_t s, bool scaled, size_t n) {
+  return align16(4 * n * s) + (scaled ? align16(4 * n) : 0);
 }
 
-// LDS one wave needs for family d (s bytes per value): its largest non-root
-// stage (items and records bounded separately) and its root stage, root
-// records staged or not
-__host__ __device__ inline size_t fam_lds_bytes(const FamDev& d, size_t s, bool scaled, bool fwd, bool root_recs) {
-  const size_t nr = root_recs ? d.root_recs : 0;
-  const size_t a = fwd ? fwd_stage_bytes(s, scaled, d.max_items, d.max_recs) : bwd_stage_bytes(s, d.max_items, d.max_recs);
-  const size_t b = fwd ? fwd_root_bytes(s, scaled, d.n_clades, nr) : bwd_root_bytes(s, d.n_clades, nr);
+//   the root's terms and slots, staged behind its arrays when they fit:
+//                         operands, coefficients [nt] | slots, 8 bytes each [ns]
+__host__ __device__ inline size_t root_stage_bytes(size_t s, size_t nt, size_t ns) {
+  return align16(4 * nt) + align16(s * nt) + 8 * ns;
+}
+
+// LDS family d needs (s bytes per value): its largest non-root stage and its
+// root, with the root's terms staged or not
+__host__ __device__ inline size_t fam_lds_bytes(const FamDev& d, size_t s, bool scaled, bool fwd, int team,
+                                                bool staged) {
+  const size_t a = fwd ? fwd_bytes(s, scaled, d.max_items) : bwd_stage_bytes(s, d.max_items, (d.max_slots + team - 1) / team);
+  size_t b = fwd ? fwd_bytes(s, scaled, d.n_clades) : bwd_root_bytes(s, scaled, d.n_clades);
+  if (staged) b += root_stage_bytes(s, (fwd ? 1 : 2) * (size_t)d.root_recs, fwd ? d.root_nfs : d.root_nbs);
   return a > b ? a : b;
 }
 
-// The pooled launch (k_pool): one workgroup of kPoolWaves waves per compute
-// unit; after the shared area, a header (lock and page bitmap) and a pool of
-// kPage-byte pages from which each family takes what both its directions need.
-constexpr int kPoolWaves = 12;
-constexpr uint32_t kPage = 512;
-constexpr uint32_t kPoolHdrBytes = 256;  // lock + bitmap of up to 2016 pages
-// bytes a family takes from the pool: the root records are staged when that
-// costs at most an eighth of the pool more
-__host__ __device__ inline size_t pool_need(const FamDev& d, size_t s, bool scaled, size_t pool_bytes) {
-  const size_t w0 = fam_lds_bytes(d, s, scaled, true, false), w1 = fam_lds_bytes(d, s, scaled, false, false);
-  const size_t r0 = fam_lds_bytes(d, s, scaled, true, true), r1 = fam_lds_bytes(d, s, scaled, false, true);
-  const size_t without = w0 > w1 ? w0 : w1, with = r0 > r1 ? r0 : r1;
-  return (with <= pool_bytes && with - without <= pool_bytes / 8) ? with : without;
-}
-
-// LDS of one launch of k_forward / k_backward: every wave of a workgroup runs
-// its own family in `wave_bytes` of LDS (laid out per stage); `shared_bytes`
-// (slice tables, reverse-sweep accumulators, node constants) come first and
-// are shared by the workgroup's waves.
+// A launch of k_forward / k_backward: every family of a workgroup has
+// `wave_bytes` of LDS (laid out per stage); `shared_bytes` (control words,
+// reverse-sweep accumulators, node constants) come first and are
+// shared by the workgroup.
 struct LdsCfg {
   uint32_t wave_bytes;
   uint32_t shared_bytes;
 };
 
-// a launch: `fpw` families (waves) per workgroup, slice tables in LDS or not.
-// With `gws` the waves' stage buffers (wave_bytes each) live in a global
-// workspace instead of LDS, one wave per workgroup: the path of families whose
-// largest stage does not fit one compute unit's LDS.
+// a launch: `fpw` families of one wave each per workgroup, or one family of
+// `team` waves.  With `gws` the families' stage
+// buffers (wave_bytes each) live in a global workspace instead of LDS, one
+// family per workgroup: the path of families whose largest stage does not fit
+// one compute unit's LDS.
 struct LaunchCfg {
   int grid = 1;
   int fpw = 1;
-  int waves_per_cu = 0;  // resident waves per compute unit the LDS allows
-  bool tabl = false;
+  int team = 1;
+  int waves_per_cu = 0;  // families per compute unit the LDS allows
   bool gws = false;
   LdsCfg L{};
   size_t lds() const { return (size_t)L.shared_bytes + (gws ? 0 : (size_t)fpw * L.wave_bytes); }
   size_t gws_bytes() const { return gws ? (size_t)grid * fpw * L.wave_bytes : 0; }
 };
 
-size_t fwd_shared_bytes(int mode, bool tabl, int tab_rows, int n, int nwgd);
-size_t bwd_shared_bytes(int mode, bool tabl, int tab_rows, int acc_n, int n, int nwgd);
+constexpr size_t kCtlBytes = 16 + 32 * kMaxTeam;  // control words and the waves' partial sums of a workgroup
+// the gradient's accumulators in LDS (0: too many, they are added to global memory)
+__host__ __device__ inline size_t acc_lds_bytes(int n) { return n <= 4096 ? align16(8 * (size_t)n) : 0; }
+size_t fwd_shared_bytes(int mode, int n, int nwgd);
+size_t bwd_shared_bytes(int mode, int n, int nwgd);
 
 // forward/backward launch: `mode` is WHALE_FP64_PLAIN / WHALE_FP32_SCALED /
-// WHALE_FP64_SCALED; fam_single >= 0 runs that one family (first wave of a
-// 1-block grid), otherwise waves take families order[fam_begin .. fam_end)
+// WHALE_FP64_SCALED; fam_single >= 0 runs that one family (first family of a
+// 1-block grid), otherwise waves or teams take families order[fam_begin .. fam_end)
 // from the ticket.  fam_count, if not null, replaces fam_end with a count read
 // on the device (the FP64 pass over families listed by the FP32 pass).
 // One component of a mixture launch: with K components the grid is K times
@@ -172,6 +181,20 @@ struct MixComp {
 };
 constexpr int kMaxMix = 8;
 
+// the launches of one arithmetic (dp.hpp; instantiated in dp_*.hip)
+template <typename R, bool S>
+hipError_t fwd_variant(bool store_all, const LaunchCfg& C, hipStream_t st, const BatchDev& B, const ModelDev& M,
+                       const WorkRaw& W, int32_t fam_single, uint32_t fam_begin, uint32_t fam_end,
+                       const uint32_t* fam_count, const MixComp* X, int K);
+template <typename R, bool S>
+hipError_t bwd_variant(const LaunchCfg& C, hipStream_t st, const BatchDev& B, const ModelDev& M, const WorkRaw& W,
+                       int32_t fam_single, uint32_t fam_begin, uint32_t fam_end, const uint32_t* fam_count,
+                       const MixComp* X, int K);
+struct FusedSlots;
+template <typename R, bool S>
+hipError_t fused_variant(const LaunchCfg& C, hipStream_t st, const BatchDev& B, const ModelDev& M, const WorkRaw& W,
+                         uint32_t fam_begin, uint32_t fam_end, const uint32_t* fam_count, int grad,
+                         const FusedSlots& SL);
 hipError_t launch_forward(int mode, bool store_all, const LaunchCfg& C, hipStream_t st, const BatchDev& B,
                           const ModelDev& M, const WorkRaw& W, int32_t fam_single, uint32_t fam_begin,
                           uint32_t fam_end, const uint32_t* fam_count = nullptr, const MixComp* X = nullptr,
@@ -185,30 +208,24 @@ hipError_t launch_backward(int mode, const LaunchCfg& C, hipStream_t st, const B
 // (−inf if not finite); resp (n_fam × K, may be null) = r
 hipError_t launch_mix(hipStream_t st, const MixComp* X, int K, const double* log_prior, uint32_t n_fam, int cond,
                       double* out, double* resp);
-// per-wave slots of the fused forward + reverse launch: each holds one
-// family's stored rows (from byte 0), ī (from ibar_off) and record
-// coefficients (from coef_off)
+// per-family slots of the fused forward + reverse launch: each holds one
+// family's stored rows (from byte 0), ī (from ibar_off) and its items'
+// exponents (from eit_off)
 struct FusedSlots {
   unsigned char* base = nullptr;
   uint64_t slot_bytes = 0;
   uint64_t ibar_off = 0;
-  uint64_t coef_off = 0;
+  uint64_t eit_off = 0;
 };
 hipError_t launch_fused(int mode, const LaunchCfg& C, hipStream_t st, const BatchDev& B, const ModelDev& M,
                         const WorkRaw& W, uint32_t fam_begin, uint32_t fam_end, const uint32_t* fam_count, int grad,
                         const FusedSlots& SL);
-// the pooled launch over families order[fam_begin .. fam_end): C.grid
-// workgroups of kPoolWaves waves, C.L.shared_bytes of shared LDS (the reverse
-// sweep's layout, tables in LDS) and C.L.wave_bytes of pool (header included)
-hipError_t launch_pool(int mode, bool store_all, const LaunchCfg& C, hipStream_t st, const BatchDev& B,
-                       const ModelDev& M, const WorkRaw& W, uint32_t fam_begin, uint32_t fam_end, int grad);
-hipError_t launch_tables(hipStream_t st, const ModelDev& M, double* eps, double* phi, double* psi, double* drow,
-                         double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels);
+hipError_t launch_tables(hipStream_t st, const ModelDev& M, double* eps, double* phi, double* psi, double* pack64,
+                         float* pack32, double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels);
 // n_eff (null: n_fam) holds the family count the conditioning term's
 // derivative is scaled by (Σ of the reverse sweep's family weights)
 hipError_t launch_tail(hipStream_t st, const ModelDev& M, const double* fam_ll, uint32_t n_fam, const double* acc,
-                       double* ebar, const double* drow, const double* dnode, const int32_t* dlevels,
-                       const int32_t* dnodes, int n_dlevels, int cond, int with_grad, double* out,
+                       double* ebar, const int32_t* dlevels, const int32_t* dnodes, int n_dlevels, int cond, int with_grad, double* out,
                        const double* n_eff = nullptr);
 hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, int n);
 hipError_t launch_det_sum(hipStream_t st, const double* slots, uint32_t n_fam, int ncol, double* out);

@@ -240,19 +240,53 @@ namespace {
 
 struct FamPlan {
   std::string err;
-  uint32_t n_clades = 0, max_items = 0, max_recs = 0, root_recs = 0;
-  std::vector<StageDev> stage;      // item0 relative to family, seg0 relative
+  uint32_t n_clades = 0, max_items = 0, max_slots = 0, n_items = 0;
+  std::vector<StageDev> stage;      // item0, seg0 and slots relative to the family
   std::vector<SegDev> seg;          // ell/ibar relative to family
-  uint32_t root_seg = 0, root_item0 = 0;
-  std::vector<uint32_t> it_seg, it_gid, it_rec;  // it_seg, it_rec family-relative
-  std::vector<int32_t> it_cf, it_cg, it_bar;
-  std::vector<uint32_t> rec_ops, rec_sid;
-  std::vector<uint16_t> rec_own;                              // stage-local item owning each record
-  std::vector<uint32_t> lvl;
+  uint32_t root_seg = 0, root_fs = 0, root_bs = 0, root_recs = 0;
+  std::vector<uint32_t> it_seg, it_gid;  // it_seg family-relative
+  std::vector<uint32_t> fs4, fs2, bs4, bs2, rec_ops, rec_sid, ent_ops, ent_rec;
+  std::vector<uint32_t> lvl_f, lvl_b;
   uint64_t ell = 0, ibar = 0;
   int64_t cells = 0, split_terms = 0, sum_compat = 0, row_steps = 0;
   double cost = 0;
 };
+
+// lanes of an item with `terms` terms
+uint32_t slot_lanes(uint32_t terms) {
+  return std::max(1u, std::min(kSlotLanes, (terms + kSlotRecs - 1) / kSlotRecs));
+}
+
+// Deals items to slots (plan.hpp): item k of `items` has cnt[k] terms and
+// takes one lane, or up to kSlotLanes adjacent lanes of a 16-lane row when it
+// has more than kSlotRecs.  Items with the most terms come first, so that the
+// 64 lanes of a chunk have similar counts; the lanes a many-lane item leaves
+// at the end of a row go to one-lane items.
+// Rows are counted from `offset` slots before the first.
+// Returns per lane (k, position) or (-1, 0) for an unused lane.
+std::vector<std::pair<int, uint32_t>> deal_slots(const std::vector<uint32_t>& cnt, uint32_t offset) {
+  const int n = (int)cnt.size();
+  std::vector<int> by(n);
+  std::iota(by.begin(), by.end(), 0);
+  std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return cnt[a] > cnt[b]; });
+  std::vector<std::pair<int, uint32_t>> out;
+  std::vector<uint32_t> holes;
+  size_t next_hole = 0;
+  for (int k : by) {
+    const uint32_t u = slot_lanes(cnt[k]);
+    if (u == 1 && next_hole < holes.size()) {
+      out[holes[next_hole++]] = {k, 0};
+      continue;
+    }
+    if ((out.size() + offset) % kSlotLanes + u > kSlotLanes)
+      while ((out.size() + offset) % kSlotLanes) {
+        holes.push_back((uint32_t)out.size());
+        out.push_back({-1, 0});
+      }
+    for (uint32_t j = 0; j < u; ++j) out.push_back({k, j});
+  }
+  return out;
+}
 
 void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int32_t* leaf_sp,
                  const int64_t* soff, const int32_t* g1, const int32_t* g2, FamPlan& F) {
@@ -454,12 +488,10 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
     idx[e].assign(nc, -1);
     for (size_t j = 0; j < comp[e].size(); ++j) idx[e][comp[e][j]] = (int32_t)j;
   }
-  // items, records, inverse records
-  auto emit_stage = [&](const std::vector<int>& segs, bool is_root) {
-    StageDev sd{};
-    sd.item0 = (uint32_t)F.it_seg.size();
-    sd.seg0 = (uint32_t)segof[segs[0]];
-    sd.n_segs = (uint32_t)segs.size();
+  // A stage's items, records and slots.  Records and entries come item by
+  // item, so an item's terms are contiguous and a slot is a range of them.
+  std::vector<uint32_t> r0, ne, e0, cnt;
+  auto emit_items = [&](const std::vector<int>& segs, StageDev& sd) -> bool {
     uint32_t local = 0;
     for (int e : segs) {
       SegDev& s = F.seg[segof[e]];
@@ -467,81 +499,136 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
       local += s.nc;
       sd.r_max = std::max(sd.r_max, s.R);
     }
+    sd.item0 = (uint32_t)F.it_seg.size();
+    sd.seg0 = (uint32_t)segof[segs[0]];
+    sd.n_segs = (uint32_t)segs.size();
     sd.n_items = local;
-    if (local > 0xffff) { F.err = "stage with more than 65535 items"; return sd; }
-    if (!is_root) F.max_items = std::max(F.max_items, local);
+    if (local > 0xffff) { F.err = "stage with more than 65535 items"; return false; }
+    const uint32_t rb = (uint32_t)F.rec_ops.size();
+    r0.assign(local + 1, 0);
     for (int e : segs) {
       const SegDev& s = F.seg[segof[e]];
-      const NodeDev& nd = m.nodes[e];
-      int par = nd.parent;
-      int slot = -1;
-      if (par >= 0) slot = (m.nodes[par].child0 == e) ? 0 : 1;
       for (uint32_t j = 0; j < s.nc; ++j) {
-        int gid = comp[e][j];
-        uint32_t me = s.item0 + j;
+        const int gid = comp[e][j];
         F.it_seg.push_back((uint32_t)segof[e]);
         F.it_gid.push_back((uint32_t)gid);
-        F.it_rec.push_back((uint32_t)F.rec_ops.size());
-        int32_t cfv = -1, cgv = -1;
-        int kids[2] = {nd.child0, nd.child1};
-        for (int k = 0; k < 2; ++k) {
-          int ch = kids[k];
-          if (ch < 0 || segof[ch] < 0) continue;
-          int x = idx[ch][gid];
-          if (x < 0) continue;
-          const SegDev& cs = F.seg[segof[ch]];
-          int32_t cell = (int32_t)(cs.ell + (uint64_t)(cs.R - 1) * cs.nc + x);
-          (k == 0 ? cfv : cgv) = cell;
-        }
-        F.it_cf.push_back(cfv);
-        F.it_cg.push_back(cgv);
-        if (is_root) F.it_bar.push_back(-1);
-        else {
-          const SegDev& ps = F.seg[segof[par]];
-          int x = idx[par][gid];
-          if (x < 0) { F.err = "internal error: clade not compatible with the parent"; return sd; }
-          F.it_bar.push_back((int32_t)(ps.ibar + (uint64_t)slot * ps.nc + x));
-        }
+        r0[s.item0 + j] = (uint32_t)F.rec_ops.size();
         for (int64_t k = soff[gid]; k < soff[gid + 1]; ++k) {
-          uint32_t l1 = s.item0 + (uint32_t)idx[e][g1[k]], l2 = s.item0 + (uint32_t)idx[e][g2[k]];
-          uint32_t r = (uint32_t)F.rec_ops.size();
+          const uint32_t l1 = s.item0 + (uint32_t)idx[e][g1[k]], l2 = s.item0 + (uint32_t)idx[e][g2[k]];
           F.rec_ops.push_back(l1 | (l2 << 16));
           F.rec_sid.push_back((uint32_t)(k - soff[0]));
-          F.rec_own.push_back((uint16_t)me);
         }
       }
     }
-    {
-      uint32_t nrec = (uint32_t)F.rec_ops.size() - F.it_rec[sd.item0];
-      sd.rec0 = F.it_rec[sd.item0];
-      sd.n_recs = nrec;
-      if (is_root) F.root_recs = nrec;
-      else F.max_recs = std::max(F.max_recs, nrec);
+    const uint32_t re = (uint32_t)F.rec_ops.size();
+    r0[local] = re;
+    // the same splits listed by part: (owner, other part, record)
+    ne.assign(local + 1, 0);
+    for (uint32_t r = rb; r < re; ++r) ++ne[F.rec_ops[r] & 0xffff], ++ne[F.rec_ops[r] >> 16];
+    e0.assign(local + 1, 0);
+    e0[0] = 2 * rb;
+    for (uint32_t i = 0; i < local; ++i) e0[i + 1] = e0[i] + ne[i];
+    F.ent_ops.resize(2 * (size_t)re);
+    F.ent_rec.resize(2 * (size_t)re);
+    std::vector<uint32_t> at(e0.begin(), e0.end() - 1);
+    for (uint32_t i = 0; i < local; ++i)
+      for (uint32_t r = r0[i]; r < r0[i + 1]; ++r) {
+        const uint32_t x = F.rec_ops[r] & 0xffff, y = F.rec_ops[r] >> 16;
+        F.ent_ops[at[x]] = i | (y << 16), F.ent_rec[at[x]++] = r;
+        F.ent_ops[at[y]] = i | (x << 16), F.ent_rec[at[y]++] = r;
+      }
+    return true;
+  };
+  // slots of the items [lo, hi) of the stage, in one direction
+  auto emit_slots = [&](const StageDev& sd, uint32_t lo, uint32_t hi, bool fwd, uint32_t offset) -> bool {
+    const std::vector<uint32_t>& off = fwd ? r0 : e0;
+    std::vector<uint32_t>&s4 = fwd ? F.fs4 : F.bs4, &s2 = fwd ? F.fs2 : F.bs2;
+    cnt.resize(hi - lo);
+    for (uint32_t i = lo; i < hi; ++i) {
+      cnt[i - lo] = off[i + 1] - off[i];
+      if (cnt[i - lo] > kSlotLanes * 0xffffu) { F.err = "clade with too many splits"; return false; }
     }
-    return sd;
+    for (const auto& [k, pos] : deal_slots(cnt, offset)) {
+      if (k < 0) {
+        s4.insert(s4.end(), {0xffffffffu, 0xffffffffu, 0u, 0u});
+        s2.insert(s2.end(), {0u, 0u});
+        continue;
+      }
+      const uint32_t i = lo + (uint32_t)k, terms = cnt[k];
+      const uint32_t u = slot_lanes(terms);
+      const uint32_t a = (uint32_t)((uint64_t)terms * pos / u), b = (uint32_t)((uint64_t)terms * (pos + 1) / u);
+      const uint32_t si = F.it_seg[sd.item0 + i], gid = F.it_gid[sd.item0 + i];
+      const int e = (int)F.seg[si].node;
+      const NodeDev& nd = m.nodes[e];
+      int32_t kc[2] = {-1, -1};
+      const int kids[2] = {nd.child0, nd.child1};
+      for (int q = 0; q < 2; ++q) {
+        const int ch = kids[q];
+        if (ch < 0 || segof[ch] < 0 || idx[ch][gid] < 0) continue;
+        const SegDev& cs = F.seg[segof[ch]];
+        kc[q] = (int32_t)(cs.ell + (uint64_t)(cs.R - 1) * cs.nc + idx[ch][gid]);
+      }
+      if (nd.kind == WHALE_NODE_WGD) kc[1] = kc[0];
+      uint32_t d;
+      if (fwd) {
+        d = gid | ((si - sd.seg0) << 16);
+      } else if (nd.parent < 0) {
+        d = 0;
+      } else {
+        const SegDev& ps = F.seg[segof[nd.parent]];
+        const int x = idx[nd.parent][gid];
+        if (x < 0) { F.err = "internal error: clade not compatible with the parent"; return false; }
+        d = ps.ibar + (m.nodes[nd.parent].child0 == e ? 0u : ps.nc) + (uint32_t)x;
+      }
+      s4.insert(s4.end(), {(uint32_t)kc[0], (uint32_t)kc[1], i | (pos << 16) | (pos + 1 == u ? kSlotLead : 0u), d});
+      s2.insert(s2.end(), {off[i] + a, (b - a) | (fwd ? 0u : (si - sd.seg0) << 16)});
+    }
+    return true;
   };
   for (auto& st : stages) {
-    StageDev sd = emit_stage(st, false);
-    if (!F.err.empty()) return;
+    StageDev sd{};
+    if (!emit_items(st, sd)) return;
+    if (sd.n_segs > 0xffff) { F.err = "stage with more than 65535 segments"; return; }
+    sd.fs0 = (uint32_t)(F.fs4.size() / 4);
+    sd.bs0 = (uint32_t)(F.bs4.size() / 4);
+    if (!emit_slots(sd, 0, sd.n_items, true, 0) || !emit_slots(sd, 0, sd.n_items, false, 0)) return;
+    sd.n_fs = (uint32_t)(F.fs4.size() / 4) - sd.fs0;
+    sd.n_bs = (uint32_t)(F.bs4.size() / 4) - sd.bs0;
+    F.max_items = std::max(F.max_items, sd.n_items);
+    F.max_slots = std::max({F.max_slots, sd.n_fs, sd.n_bs});
     F.stage.push_back(sd);
   }
-  F.root_item0 = (uint32_t)F.it_seg.size();
-  StageDev rsd = emit_stage({m.root}, true);
-  if (!F.err.empty()) return;
-  (void)rsd;
-  // root levels: runs of clades in size order of which none is a part of
-  // another, so a level reads only finished parts.  Clades of one size never
-  // are; a run goes on past a size until a clade has a part inside it.
-  F.lvl.push_back(0);
-  for (int c = 1, start = 0; c < nc; ++c) {
-    int32_t dep = -1;
-    for (int64_t k = soff[c]; k < soff[c + 1]; ++k) dep = std::max(dep, std::max(g1[k], g2[k]));
-    if (dep >= start) {
-      F.lvl.push_back((uint32_t)c);
-      start = c;
+  F.n_items = (uint32_t)F.it_seg.size();
+  {
+    StageDev sd{};
+    const size_t rec_before = F.rec_ops.size();
+    if (!emit_items({m.root}, sd)) return;
+    F.root_recs = (uint32_t)(F.rec_ops.size() - rec_before);
+    // root levels: runs of clades in size order of which none is a part of
+    // another, so a level reads only finished parts (and, in the reverse
+    // sweep, only finished owners).  Clades of one size never are; a run goes
+    // on past a size until a clade has a part inside it.
+    std::vector<uint32_t> lvl{0};
+    for (int c = 1, start = 0; c < nc; ++c) {
+      int32_t dep = -1;
+      for (int64_t k = soff[c]; k < soff[c + 1]; ++k) dep = std::max(dep, std::max(g1[k], g2[k]));
+      if (dep >= start) {
+        lvl.push_back((uint32_t)c);
+        start = c;
+      }
+    }
+    lvl.push_back((uint32_t)nc);
+    F.root_fs = (uint32_t)(F.fs4.size() / 4);
+    F.root_bs = (uint32_t)(F.bs4.size() / 4);
+    for (size_t L = 0; L < lvl.size(); ++L) {
+      F.lvl_f.push_back((uint32_t)(F.fs4.size() / 4) - F.root_fs);
+      F.lvl_b.push_back((uint32_t)(F.bs4.size() / 4) - F.root_bs);
+      if (L + 1 == lvl.size()) break;
+      if (!emit_slots(sd, lvl[L], lvl[L + 1], true, F.lvl_f.back()) ||
+          !emit_slots(sd, lvl[L], lvl[L + 1], false, F.lvl_b.back()))
+        return;
     }
   }
-  F.lvl.push_back((uint32_t)nc);
   // workload counts (the reference's cell and split-term counts)
   for (auto& s : F.seg) {
     F.cells += (int64_t)s.R * s.nc;
@@ -557,7 +644,7 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
     }
   }
   F.split_terms += 2 * (soff[nc] - soff[0]);
-  uint64_t steps = 1 + F.lvl.size();
+  uint64_t steps = 1 + F.lvl_f.size();
   for (auto& sd : F.stage) steps += sd.r_max;
   F.cost = (double)steps * 64.0 + (double)F.cells + (double)F.split_terms;
 }
@@ -582,7 +669,7 @@ std::string build_plan(const ModelHost& m, int n_fam, const int64_t* fam_clade_o
   for (auto& t : th) t.join();
   for (int f = 0; f < n_fam; ++f)
     if (!fp[f].err.empty()) return "family " + std::to_string(f) + ": " + fp[f].err;
-  // concatenate
+  // concatenate: every family's offsets first, then the copies on the same threads
   P = PlanHost();
   P.cost_order.resize(n_fam);
   std::iota(P.cost_order.begin(), P.cost_order.end(), 0u);
@@ -591,71 +678,114 @@ std::string build_plan(const ModelHost& m, int n_fam, const int64_t* fam_clade_o
   P.fam.resize(n_fam);
   P.fam_seg0.resize(n_fam);
   P.fam_nseg.resize(n_fam);
-  uint64_t ell = 0, ibar = 0;
+  uint64_t ell = 0, ibar = 0, item = 0, seg = 0, stage = 0, rec = 0, fs = 0, bs = 0, lvl = 0;
   for (int f = 0; f < n_fam; ++f) {
-    FamPlan& F = fp[f];
+    const FamPlan& F = fp[f];
     FamDev& d = P.fam[f];
-    uint32_t item_base = (uint32_t)P.it_seg.size();
-    uint32_t seg_base = (uint32_t)P.seg.size();
-    uint32_t rec_base = (uint32_t)P.rec_ops.size();
     d.n_clades = F.n_clades;
     d.n_stages = (uint32_t)F.stage.size();
-    d.stage0 = (uint32_t)P.stage.size();
-    d.root_item0 = item_base + F.root_item0;
+    d.stage0 = (uint32_t)stage;
+    d.item0 = (uint32_t)item;
+    d.n_items = F.n_items;
     d.clade0 = (uint32_t)fam_clade_off[f];
     d.split0 = (uint32_t)split_off[fam_clade_off[f]];
-    d.lvl0 = (uint32_t)P.lvl.size();
-    d.n_lvl = (uint32_t)F.lvl.size() - 1;
+    d.lvl0 = (uint32_t)lvl;
+    d.n_lvl = (uint32_t)F.lvl_f.size() - 1;
     d.max_items = F.max_items;
-    d.max_recs = F.max_recs;
+    d.max_slots = F.max_slots;
+    d.root_seg = (uint32_t)(seg + F.root_seg);
+    d.root_fs = (uint32_t)(fs + F.root_fs);
+    d.root_bs = (uint32_t)(bs + F.root_bs);
+    d.root_nfs = F.lvl_f.back();
+    d.root_nbs = F.lvl_b.back();
     d.root_recs = F.root_recs;
-    d.root_seg = seg_base + F.root_seg;
-    d.rec0 = rec_base;
+    d.rec0 = (uint32_t)rec;
     d.n_recs = (uint32_t)F.rec_ops.size();
     d.ell0 = ell;
     d.ibar0 = ibar;
-    P.fam_seg0[f] = seg_base;
+    P.fam_seg0[f] = (uint32_t)seg;
     P.fam_nseg[f] = (uint32_t)F.seg.size();
-    for (auto s : F.stage) {
-      s.item0 += item_base;
-      s.seg0 += seg_base;
-      s.rec0 += rec_base;
-      P.stage.push_back(s);
-    }
-    for (auto& s : F.seg) P.seg.push_back(s);
-    for (size_t i = 0; i < F.it_seg.size(); ++i) {
-      P.it_seg.push_back(F.it_seg[i] + seg_base);
-      P.it_gid.push_back(F.it_gid[i]);
-      P.it_rec.push_back(F.it_rec[i] + rec_base);
-      P.it_cf.push_back(F.it_cf[i]);
-      P.it_cg.push_back(F.it_cg[i]);
-      P.it_bar.push_back(F.it_bar[i]);
-    }
-    for (size_t r = 0; r < F.rec_ops.size(); ++r) {
-      P.rec_ops.push_back(F.rec_ops[r]);
-      P.rec_sid.push_back(F.rec_sid[r]);
-      P.rec_own.push_back(F.rec_own[r]);
-      P.rec_p.push_back(p[d.split0 + F.rec_sid[r]]);
-    }
-    for (auto v : F.lvl) P.lvl.push_back(v);
+    stage += F.stage.size();
+    item += F.it_seg.size();
+    seg += F.seg.size();
+    rec += F.rec_ops.size();
+    fs += F.fs4.size() / 4;
+    bs += F.bs4.size() / 4;
+    lvl += F.lvl_f.size();
     ell += F.ell;
     ibar += F.ibar;
     P.max_items = std::max(P.max_items, std::max(F.max_items, F.n_clades));
-    P.max_recs = std::max(P.max_recs, F.max_recs);
-    P.max_root_recs = std::max(P.max_root_recs, F.root_recs);
     P.cells += F.cells;
     P.split_terms += F.split_terms;
     P.sum_compat += F.sum_compat;
     P.row_steps += F.row_steps;
     P.n_clades += F.n_clades;
-    {  // release the family's temporaries, keep its cost for nothing else
-      FamPlan tmp;
-      tmp.cost = F.cost;
-      std::swap(tmp, F);
-    }
   }
-  // sentinel: it_rec of one past the last item
-  P.it_rec.push_back((uint32_t)P.rec_ops.size());
+  for (uint64_t x : {item, 2 * rec, fs, bs})
+    if (x > 0xffffffffull) return "batch too large";
+  P.stage.resize(stage);
+  P.seg.resize(seg);
+  P.run.resize(seg);
+  P.it_seg.resize(item);
+  P.it_gid.resize(item);
+  P.fs4.resize(4 * fs);
+  P.fs2.resize(2 * fs);
+  P.bs4.resize(4 * bs);
+  P.bs2.resize(2 * bs);
+  P.rec_ops.resize(rec);
+  P.rec_p.resize(rec);
+  P.ent_ops.resize(2 * rec);
+  P.ent_p.resize(2 * rec);
+  P.lvl_f.resize(lvl);
+  P.lvl_b.resize(lvl);
+  auto copy_family = [&](int f) {
+    FamPlan& F = fp[f];
+    const FamDev& d = P.fam[f];
+    const uint32_t seg0 = P.fam_seg0[f];
+    const uint32_t fs0 = d.root_fs - F.root_fs, bs0 = d.root_bs - F.root_bs;
+    for (size_t k = 0; k < F.stage.size(); ++k) {
+      StageDev s = F.stage[k];
+      s.item0 += d.item0;
+      s.seg0 += seg0;
+      s.fs0 += fs0;
+      s.bs0 += bs0;
+      P.stage[d.stage0 + k] = s;
+    }
+    for (size_t k = 0; k < F.seg.size(); ++k) {
+      const SegDev& s = F.seg[k];
+      const NodeDev& nd = m.nodes[s.node];
+      P.seg[seg0 + k] = s;
+      SegRun& t = P.run[seg0 + k];
+      t.ell = s.ell - s.item0;
+      t.nc = s.nc;
+      t.R = s.R;
+      t.tab = (uint32_t)nd.tab;
+      t.kn = (uint32_t)nd.kind | (s.node << 2);
+      t.c0 = nd.kind == WHALE_NODE_LEAF ? s.node : (uint32_t)nd.child0;
+      t.c1 = (uint32_t)(nd.kind == WHALE_NODE_WGD ? nd.wgd : nd.child1);
+      t.ibar = s.ibar - s.item0;
+    }
+    for (size_t i = 0; i < F.it_seg.size(); ++i) P.it_seg[d.item0 + i] = F.it_seg[i] + seg0;
+    std::copy(F.it_gid.begin(), F.it_gid.end(), P.it_gid.begin() + d.item0);
+    std::copy(F.fs4.begin(), F.fs4.end(), P.fs4.begin() + 4 * (size_t)fs0);
+    std::copy(F.fs2.begin(), F.fs2.end(), P.fs2.begin() + 2 * (size_t)fs0);
+    std::copy(F.bs4.begin(), F.bs4.end(), P.bs4.begin() + 4 * (size_t)bs0);
+    std::copy(F.bs2.begin(), F.bs2.end(), P.bs2.begin() + 2 * (size_t)bs0);
+    std::copy(F.rec_ops.begin(), F.rec_ops.end(), P.rec_ops.begin() + d.rec0);
+    std::copy(F.ent_ops.begin(), F.ent_ops.end(), P.ent_ops.begin() + 2 * (size_t)d.rec0);
+    for (size_t r = 0; r < F.rec_sid.size(); ++r) P.rec_p[d.rec0 + r] = p[d.split0 + F.rec_sid[r]];
+    for (size_t k = 0; k < F.ent_rec.size(); ++k)
+      P.ent_p[2 * (size_t)d.rec0 + k] = p[d.split0 + F.rec_sid[F.ent_rec[k]]];
+    std::copy(F.lvl_f.begin(), F.lvl_f.end(), P.lvl_f.begin() + d.lvl0);
+    std::copy(F.lvl_b.begin(), F.lvl_b.end(), P.lvl_b.begin() + d.lvl0);
+    F = FamPlan();
+  };
+  th.clear();
+  for (int w = 0; w < nt; ++w)
+    th.emplace_back([&, w]() {
+      for (int f = w; f < n_fam; f += nt) copy_family(f);
+    });
+  for (auto& t : th) t.join();
   P.ell_cells = ell;
   P.ibar_cells = ibar;
   int64_t nclades = fam_clade_off[n_fam];

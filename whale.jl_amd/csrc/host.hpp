@@ -40,19 +40,17 @@ struct PlanHost {
   std::vector<FamDev> fam;
   std::vector<StageDev> stage;
   std::vector<SegDev> seg;
-  std::vector<uint32_t> it_seg, it_gid, it_rec;
-  std::vector<int32_t> it_cf, it_cg, it_bar;
-  std::vector<uint32_t> rec_ops, rec_sid;
-  std::vector<uint16_t> rec_own;   // stage-local item owning each record
-  std::vector<double> rec_p;       // p of each record (the FP64 plain coefficient)
+  std::vector<SegRun> run;
+  std::vector<uint32_t> it_seg, it_gid;
+  std::vector<uint32_t> fs4, fs2, bs4, bs2;  // slots, 4 and 2 words each (plan.hpp)
+  std::vector<uint32_t> rec_ops, ent_ops;
+  std::vector<double> rec_p, ent_p;
   std::vector<uint16_t> clade_size;
   std::vector<double> split_p;
-  std::vector<uint32_t> lvl;
+  std::vector<uint32_t> lvl_f, lvl_b;
   std::vector<uint32_t> cost_order; // families by decreasing cost
   uint64_t ell_cells = 0, ibar_cells = 0;
   uint32_t max_items = 0;
-  uint32_t max_recs = 0;             // most records of any non-root stage
-  uint32_t max_root_recs = 0;        // most records of a root stage
   // workload counts
   int64_t n_clades = 0, n_splits = 0, cells = 0, split_terms = 0, sum_compat = 0, row_steps = 0;
   // per-family compat lists in the reference layout, for ℓ download:

@@ -14,13 +14,21 @@
 //            clades form the stage's items, processed row by row in lockstep.
 //            Segments that share a clade (possible only on MUL trees) are put
 //            in different stages.
-//   item     one (segment, compatible clade) pair.  Its split list (records)
-//            refers to other items of the same stage by stage-local index, so
-//            the row buffers of a stage live in LDS and every operand is an
-//            LDS gather; the reverse sweep scatters through the same records.
+//   item     one (segment, compatible clade) pair, numbered within the stage.
+//   slot     one lane's share of one item.  An item's value is a sum over its
+//            splits (forward) or over the splits it is a part of (reverse
+//            sweep); its terms are dealt to one slot, or to up to 16 adjacent
+//            lanes of a 16-lane row when there are more than kSlotRecs.  The
+//            last of them ("lead") holds the item's value.  Every sum is a
+//            gather from the stage's row buffers in LDS followed by at most
+//            four lane shifts: no atomics, and the order of the terms does not
+//            depend on the launch.  64 slots make a chunk, one wave's work in
+//            one pass; chunks are filled longest items first, so the lanes of
+//            a chunk have similar term counts.
 //   root     the last stage of every family: all clades, one row, processed
 //            in clade-size levels (the root term uses the root's own smaller
-//            clades, src/core.jl:151-158).
+//            clades, src/core.jl:151-158); its slots are listed level by
+//            level, an item's lanes within 16 slots from a multiple of 16.
 #pragma once
 #include <stdint.h>
 
@@ -45,17 +53,22 @@ struct FamDev {
   uint32_t n_clades;
   uint32_t n_stages;     // non-root stages
   uint32_t stage0;       // first stage (absolute)
-  uint32_t root_item0;   // first item of the root stage (absolute); items are stage-local from here
+  uint32_t item0;        // first item (absolute)
   uint32_t clade0;       // first clade (absolute): clade sizes, exponents
   uint32_t split0;       // first split (absolute)
-  uint32_t lvl0;         // root size-level boundaries lvl[lvl0 .. lvl0 + n_lvl] (root-stage-local items)
+  uint32_t lvl0;         // root level boundaries: lvl_f/lvl_b[lvl0 .. lvl0 + n_lvl], slots from root_fs / root_bs
   uint32_t n_lvl;
   uint32_t max_items;    // largest non-root stage (the root stage holds all n_clades)
-  uint32_t max_recs;     // most records of any non-root stage
+  uint32_t max_slots;    // most slots of any non-root stage, either direction
   uint32_t root_seg;     // absolute segment of the root
-  uint32_t root_recs;    // records of the root stage (all splits of the family)
-  uint32_t rec0;         // first record (absolute); the family's records are contiguous
+  uint32_t root_fs;      // first forward slot of the root (absolute)
+  uint32_t root_bs;      // first reverse slot of the root (absolute)
+  uint32_t root_nfs;     // the root's slots
+  uint32_t root_nbs;
+  uint32_t root_recs;    // records of the root (the family's last)
+  uint32_t rec0;         // first record (absolute); the family's records are contiguous, its entries start at 2 rec0
   uint32_t n_recs;       // records of all its stages and its root
+  uint32_t n_items;      // items of its non-root stages
   uint64_t ell0;         // first ℓ cell (absolute)
   uint64_t ibar0;        // first ī cell (absolute)
 };
@@ -66,8 +79,10 @@ struct StageDev {
   uint32_t r_max;        // largest R among its segments
   uint32_t seg0;         // absolute first segment
   uint32_t n_segs;
-  uint32_t rec0;         // absolute first record (records of its items, owner by owner)
-  uint32_t n_recs;
+  uint32_t fs0;          // absolute first forward slot
+  uint32_t n_fs;
+  uint32_t bs0;          // absolute first reverse slot
+  uint32_t n_bs;
   uint32_t pad;
 };
 
@@ -80,16 +95,36 @@ struct SegDev {
   uint32_t ibar;         // first ī cell relative to FamDev::ibar0 (slot k of child k: + k*nc), kNone if none
 };
 
-// Items: structure of arrays over all items of the batch (absolute index).
-//   it_seg[i]   absolute segment
-//   it_gid[i]   family-local clade id
-//   it_rec[i]   first record; records of item i are [it_rec[i], it_rec[i+1])
-//   it_cf[i]    ℓ cell (relative to ell0) of child0's top row for this clade, or -1
-//   it_cg[i]    same for child1
-//   it_bar[i]   ī cell (relative to ibar0) holding d logL / d top-row value, -1 at the root
-// Records (one per split of an item's clade):
-//   rec_ops[r]  l1 | l2 << 16, stage-local items of the two parts
-//   rec_sid[r]  family-local split id (p = split_p[split0 + sid])
-//   rec_own[r]  stage-local item owning the record (records of an item are contiguous)
+// what a lane needs of its item's segment and node: two 16-byte loads
+struct alignas(16) SegRun {
+  uint32_t ell;          // SegDev::ell - item0, so the cell of stage item i at row r is ell + i + r*nc (mod 2^32)
+  uint32_t nc;
+  uint32_t R;
+  uint32_t tab;          // first row of the node in the slice tables
+  uint32_t kn;           // node kind | node << 2
+  uint32_t c0;           // child0 (leaf: the node itself)
+  uint32_t c1;           // child1; a WGD node: its q index
+  uint32_t ibar;         // SegDev::ibar - item0
+};
+
+// Slots: two arrays per direction, over all slots of the batch.
+//   s4[s] = {a, b, c, d}
+//     a, b   ℓ cells (relative to ell0) of child0's and child1's top rows for
+//            the slot's clade, or -1 (a WGD node's one child stands in both)
+//     c      item | position within the item's slots << 16 | kSlotLead
+//     d      forward: clade | stage-local segment << 16
+//            reverse: ī cell (relative to ibar0) holding d logL / d top-row value
+//   s2[s] = {start, count | (reverse: stage-local segment << 16)}
+//            the slot's terms: records rec0 + start .. (forward) or entries
+//            2 rec0 + start .. (reverse)
+// Unused lanes have no terms and no lead.
+// Records (one per split of an item's clade): rec_ops[r] = l1 | l2 << 16,
+// stage-local items of the two parts; rec_p[r] = p.
+// Entries (two per record, listed by part): ent_ops[k] = owner | other << 16,
+// the stage-local items owning the record and of its other part; ent_p[k] = p.
+constexpr uint32_t kSlotLead = 1u << 20;
+constexpr uint32_t kSlotRecs = 4;       // terms a slot holds before an item takes another lane
+constexpr uint32_t kSlotLanes = 16;     // most lanes of one item
+constexpr uint32_t kChunk = 64;
 
 }  // namespace whale

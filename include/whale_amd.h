@@ -297,7 +297,7 @@ int whale_download_ell(whale_batch* b, int32_t family, double* out, int64_t cap,
 
 /* Stochastic backtracking of reconciled trees from the ℓ the last call
  * stored (backtrack(wm, ccd) after logpdf!(wm, ccd), src/track.jl:188-414),
- * on the device, one lane per (family, sample): n_samples trees for each of
+ * on the device, one wave per (family, sample): n_samples trees for each of
  * the families [family, family + n_families).  Events are drawn with the
  * reference's weights and in its order; the uniform numbers come from a
  * counter-based generator of (seed, family, sample), so a call is

@@ -2094,18 +2094,38 @@ int whale_backtrack(whale_batch* b, int32_t family, int32_t n_families, int32_t 
   const uint64_t lanes_total = (uint64_t)n_families * n_samples;
   const uint64_t fam_chunk = std::max<uint64_t>(1, (256ull << 20) / (per_lane * n_samples));
   const uint64_t lanes_cap = std::min<uint64_t>(lanes_total, fam_chunk * n_samples);
-  HIPCHK(b->bt_counts.alloc(4 * lanes_cap));
+  // per walk where its nodes were packed; the packing cursor; the node counts
+  HIPCHK(b->bt_counts.alloc(8 * (lanes_cap + 1) + 4 * lanes_cap));
   HIPCHK(b->bt_nodes.alloc(per_lane * lanes_cap));
   HIPCHK(b->bt_stack.alloc(per_lane * lanes_cap));
   for (uint64_t f0 = 0; f0 < (uint64_t)n_families; f0 += fam_chunk) {
     const uint32_t nf = (uint32_t)std::min<uint64_t>(fam_chunk, n_families - f0);
     const uint64_t lanes = (uint64_t)nf * n_samples;
-    HIPCHK(launch_backtrack(st, D, M, (uint32_t)(family + f0), nf, (uint32_t)n_samples, seed, (uint32_t)cap,
-                            b->bt_counts.as<int32_t>(), b->bt_nodes.as<int32_t>(), b->bt_stack.as<int32_t>()));
-    HIPCHK(hipMemcpyAsync(counts + f0 * n_samples, b->bt_counts.p, 4 * lanes, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(nodes + f0 * n_samples * 4 * (uint64_t)cap, b->bt_nodes.p, per_lane * lanes,
-                          hipMemcpyDeviceToHost, st));
+    uint32_t max_items = 0;
+    for (uint64_t k = 0; k < nf; ++k) max_items = std::max(max_items, P.fam[family + f0 + k].n_items);
+    uint64_t* const d_first = b->bt_counts.as<uint64_t>();
+    int32_t* const d_counts = (int32_t*)(d_first + lanes + 1);
+    HIPCHK(launch_fill_u32(st, (uint32_t*)(d_first + lanes), 0u, 2));
+    HIPCHK(launch_backtrack(st, D, M, (uint32_t)(family + f0), nf, (uint32_t)n_samples, seed, (uint32_t)cap, d_counts,
+                            b->bt_nodes.as<int32_t>(), b->bt_stack.as<int32_t>(), max_items));
+    // the nodes that the walks hold, packed where their stacks were
+    HIPCHK(launch_bt_pack(st, lanes, d_counts, b->bt_nodes.as<int32_t>(), (uint32_t)cap, d_first,
+                          d_first + lanes, b->bt_stack.as<int32_t>()));
+    std::vector<uint64_t> first(lanes + 1);
+    HIPCHK(hipMemcpyAsync(first.data(), d_first, 8 * (lanes + 1), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(counts + f0 * n_samples, d_counts, 4 * lanes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    std::vector<int32_t> packed(4 * (size_t)first[lanes]);
+    if (!packed.empty()) {
+      HIPCHK(hipMemcpyAsync(packed.data(), b->bt_stack.p, 4 * packed.size(), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+    }
+    for (uint64_t k = 0; k < lanes; ++k) {
+      const int32_t n = counts[f0 * n_samples + k];
+      if (n > 0)
+        std::memcpy(nodes + (f0 * n_samples + k) * 4 * (uint64_t)cap, packed.data() + 4 * (size_t)first[k],
+                    16 * (size_t)n);
+    }
   }
   return WHALE_OK;
 }

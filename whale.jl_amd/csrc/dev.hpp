@@ -253,7 +253,9 @@ struct BtDev {
 };
 hipError_t launch_backtrack(hipStream_t st, const BtDev& D, const ModelDev& M, uint32_t fam_begin, uint32_t n_fams,
                             uint32_t n_samples, uint64_t seed, uint32_t cap, int32_t* counts, int32_t* nodes,
-                            int32_t* stack);
+                            int32_t* stack, uint32_t max_items);
+hipError_t launch_bt_pack(hipStream_t st, uint64_t walks, const int32_t* counts, const int32_t* nodes, uint32_t cap,
+                          uint64_t* first, uint64_t* cursor, int32_t* packed);
 
 // The fixed per-GPU workspace of whale_logpdf_noalloc (a file-scope device
 // array in kernels.hip) and its device address on `device`, which must be the

@@ -231,6 +231,14 @@ struct whale_batch {
   std::vector<std::unique_ptr<MixWork>> mixw;
   DBuf mixsel, mixprior, mixout, mixresp;
   LaunchCfg cfg[3][2][kClasses];   // [mode][forward, backward][class]
+  // the launches of one evaluation: a class, or adjacent classes as one launch
+  // (plan_groups); a group's largest class names its entry of cfg and ticket
+  struct Group {
+    int cls, lane;
+    uint32_t lo, hi;   // order_host[lo, hi)
+    LaunchCfg cfg[2];  // forward, backward
+  };
+  std::vector<Group> groups[3];
   LaunchCfg cfg_fb[2];             // FP64 pass over families the FP32 form could not represent
   int last_mode = -1;
   int last_launch = WHALE_LAUNCH_BATCHED;
@@ -926,6 +934,86 @@ bool fits_lds(const whale_batch* b, const FamDev& d) {
   return f <= lim && r <= lim;
 }
 
+// The launches of one evaluation.  Launches on one stream run one after the
+// other, and a family takes as long alone as beside others, so a batch that
+// the GPU holds at once runs as few launches as leave it resident: adjacent
+// classes share a launch (by the largest's team; a smaller family's idle waves
+// wait at barriers) while the waves and the LDS of all families stay within
+// kFill times what the compute units hold.  Larger batches keep their classes,
+// each of which fills the GPU.  Measured, classes apart -> together, per pass:
+// 100 families, FP64 gradient, 818 -> 500 us; 1000 families, FP32 gradient,
+// 1990 -> 1310 us (1.6 times what the GPU holds; by kFill 1 in four launches
+// 1760); 777 families of 50 taxa, scaled FP64, 3350 -> 2200 us (kFill 1: 3140).
+// Past kFill the idle waves cost more than the launches: 5000 families, 2.5
+// times what the GPU holds, 3160 us apart, 3690 in two launches.
+void plan_groups(whale_batch* b, int mode) {
+  const whale_model* m = b->model;
+  std::vector<whale_batch::Group>& out = b->groups[mode];
+  out.clear();
+  const uint32_t* ord = b->order_host.data();
+  for (int j = 0; j < whale_batch::kClasses; ++j) {
+    const int k = kLayoutOrder[b->tune.layout][j];
+    if (b->cls_hi[k] > b->cls_lo[k])
+      out.push_back({k, kLayoutLane[b->tune.layout][k], b->cls_lo[k], b->cls_hi[k], {b->cfg[mode][0][k], b->cfg[mode][1][k]}});
+  }
+  std::vector<whale_batch::Group> cls = out;  // largest class first, as in order_host
+  std::sort(cls.begin(), cls.end(), [](const auto& x, const auto& y) { return x.cls > y.cls; });
+  const int nc = (int)cls.size();
+  constexpr double kFill = 2.0;
+  const double waves = kFill * m->ctx->n_cu * (mode == WHALE_FP32_SCALED ? 16 : 12);
+  const double lds = kFill * (double)m->ctx->n_cu * (double)m->ctx->lds_cu;
+  // waves and LDS of a launch's families
+  auto load = [&](const whale_batch::Group& g, double* w, double* l) {
+    for (int d = 0; d < 2; ++d) {
+      const double n = (double)(g.hi - g.lo);
+      w[d] += n * g.cfg[d].team;
+      l[d] += n * (double)g.cfg[d].lds() / g.cfg[d].fpw;
+    }
+  };
+  auto fits = [&](const std::vector<whale_batch::Group>& gs, double* total) {
+    double w[2] = {0, 0}, l[2] = {0, 0};
+    for (const auto& g : gs) load(g, w, l);
+    *total = w[0];
+    return std::max(w[0], w[1]) <= waves && std::max(l[0], l[1]) <= lds;
+  };
+  double total;
+  if (nc < 2 || !fits(cls, &total)) return;
+  // launches of classes i..j (largest first), planned when first asked for
+  std::vector<whale_batch::Group> range((size_t)nc * nc);
+  std::vector<char> known((size_t)nc * nc, 0);
+  std::vector<whale_batch::Group> best;
+  double best_total = 0;
+  for (uint32_t cut = 0; cut < 1u << (nc - 1); ++cut) {  // bit i: a launch ends after class i
+    const size_t n = (size_t)__builtin_popcount(cut) + 1;
+    if (!best.empty() && n > best.size()) continue;
+    std::vector<whale_batch::Group> gs;
+    bool ok = true;
+    for (int i = 0, j; i < nc && ok; i = j + 1) {
+      for (j = i; j < nc - 1 && !(cut >> j & 1); ++j) {}
+      whale_batch::Group& g = range[(size_t)i * nc + j];
+      char& state = known[(size_t)i * nc + j];
+      if (!state) {
+        g = cls[i];
+        g.hi = cls[j].hi;
+        state = 1;
+        if (j > i)
+          for (int d = 0; d < 2; ++d)
+            if (!plan_families(b, d == 0, mode, ord + g.lo, g.hi - g.lo, g.hi - g.lo, true, &g.cfg[d]) || g.cfg[d].gws) state = 2;
+      }
+      ok = state == 1;
+      gs.push_back(g);
+    }
+    if (!ok || !fits(gs, &total)) continue;
+    if (best.empty() || n < best.size() || total < best_total) {
+      best = gs;
+      best_total = total;
+    }
+  }
+  if (best.empty() || (int)best.size() == nc) return;
+  out = best;
+  for (size_t g = 0; g < out.size(); ++g) out[g].lane = (int)g % 3;
+}
+
 // launch shapes of every class, mode and direction, and of the FP64 pass over
 // families the FP32 form could not represent
 int plan_batch_launches(whale_batch* b) {
@@ -943,6 +1031,7 @@ int plan_batch_launches(whale_batch* b) {
         if (!plan_families(b, dir == 0, mode, b->order_host.data() + lo, hi - lo, hi - lo, true, &b->cfg[mode][dir][k]))
           return fail(WHALE_EINVAL, "a family's largest stage does not fit the LDS of one compute unit");
       }
+  for (int mode = 0; mode < 3; ++mode) plan_groups(b, mode);
   for (int dir = 0; dir < 2; ++dir)
     if (!plan_families(b, dir == 0, WHALE_FP64_SCALED, b->order_host.data(), b->order_host.size(),
                        (uint64_t)m->ctx->n_cu, false, &b->cfg_fb[dir]))
@@ -1180,12 +1269,9 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   auto batched = [&](int dir) -> int {
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
-    // classes in launch order and their streams
-    const int* kOrder = kLayoutOrder[b->tune.layout];
-    auto lane_of = [&](int k) { return kLayoutLane[b->tune.layout][k]; };
+    const std::vector<whale_batch::Group>& groups = b->groups[mode];
     bool used[kLanes] = {};
-    for (int k = 0; k < whale_batch::kClasses; ++k)
-      if (b->cls_hi[k] > b->cls_lo[k]) used[lane_of(k)] = true;
+    for (const auto& g : groups) used[g.lane] = true;
     HIPCHK(hipEventRecord(c->fork[3 * dir], st));
     for (int l = 1; l < kLanes; ++l)
       if (used[l]) HIPCHK(hipStreamWaitEvent(lanes[l], c->fork[3 * dir], 0));
@@ -1196,15 +1282,11 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
       if (dir == 0) HIPCHK(launch_forward(mode, store_all, C, st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
       else HIPCHK(launch_backward(mode, C, st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
     }
-    for (int j = 0; j < whale_batch::kClasses; ++j) {
-      const int k = kOrder[j];
-      if (b->cls_hi[k] == b->cls_lo[k]) continue;
-      hipStream_t sk = lanes[lane_of(k)];
+    for (const auto& g : groups) {
       WorkRaw Wk = W;
-      Wk.ticket = W.ticket + whale_batch::kClasses * dir + k;
-      const LaunchCfg& C = b->cfg[mode][dir][k];
-      if (dir == 0) HIPCHK(launch_forward(mode, store_all, C, sk, B, M, Wk, -1, b->cls_lo[k], b->cls_hi[k]));
-      else HIPCHK(launch_backward(mode, C, sk, B, M, Wk, -1, b->cls_lo[k], b->cls_hi[k]));
+      Wk.ticket = W.ticket + whale_batch::kClasses * dir + g.cls;
+      if (dir == 0) HIPCHK(launch_forward(mode, store_all, g.cfg[0], lanes[g.lane], B, M, Wk, -1, g.lo, g.hi));
+      else HIPCHK(launch_backward(mode, g.cfg[1], lanes[g.lane], B, M, Wk, -1, g.lo, g.hi));
     }
     for (int l = 1; l < kLanes; ++l)
       if (used[l]) {
@@ -1221,11 +1303,9 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   auto interleaved = [&]() -> int {
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
-    const int* kOrder = kLayoutOrder[b->tune.layout];
-    const int* kLane = kLayoutLane[b->tune.layout];
+    const std::vector<whale_batch::Group>& groups = b->groups[mode];
     bool used[kLanes] = {};
-    for (int k = 0; k < whale_batch::kClasses; ++k)
-      if (b->cls_hi[k] > b->cls_lo[k]) used[kLane[k]] = true;
+    for (const auto& g : groups) used[g.lane] = true;
     HIPCHK(hipEventRecord(c->fork[0], st));
     for (int l = 1; l < kLanes; ++l)
       if (used[l]) HIPCHK(hipStreamWaitEvent(lanes[l], c->fork[0], 0));
@@ -1235,25 +1315,19 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
       Wh.ticket = W.ticket + kTicketHbm;
       HIPCHK(launch_forward(mode, store_all, b->cfg_hbm[mode][0], st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
     }
-    for (int j = 0; j < whale_batch::kClasses; ++j) {
-      const int k = kOrder[j];
-      if (b->cls_hi[k] == b->cls_lo[k]) continue;
-      hipStream_t sk = lanes[kLane[k]];
+    for (const auto& g : groups) {
       WorkRaw Wk = W;
-      Wk.ticket = W.ticket + k;
-      HIPCHK(launch_forward(mode, store_all, b->cfg[mode][0][k], sk, B, M, Wk, -1, b->cls_lo[k], b->cls_hi[k]));
+      Wk.ticket = W.ticket + g.cls;
+      HIPCHK(launch_forward(mode, store_all, g.cfg[0], lanes[g.lane], B, M, Wk, -1, g.lo, g.hi));
     }
     if (hbm) {
       Wh.ticket = W.ticket + kTicketHbm + 1;
       HIPCHK(launch_backward(mode, b->cfg_hbm[mode][1], st, B, M, Wh, -1, b->hbm_lo, b->hbm_hi));
     }
-    for (int j = 0; j < whale_batch::kClasses; ++j) {
-      const int k = kOrder[j];
-      if (b->cls_hi[k] == b->cls_lo[k]) continue;
-      hipStream_t sk = lanes[kLane[k]];
+    for (const auto& g : groups) {
       WorkRaw Wk = W;
-      Wk.ticket = W.ticket + whale_batch::kClasses + k;
-      HIPCHK(launch_backward(mode, b->cfg[mode][1][k], sk, B, M, Wk, -1, b->cls_lo[k], b->cls_hi[k]));
+      Wk.ticket = W.ticket + whale_batch::kClasses + g.cls;
+      HIPCHK(launch_backward(mode, g.cfg[1], lanes[g.lane], B, M, Wk, -1, g.lo, g.hi));
     }
     for (int l = 1; l < kLanes; ++l)
       if (used[l]) {

@@ -1281,9 +1281,7 @@ struct BwdLane {
 // absolute items less it_base), writing ī through `ibar` (relative cells).
 //
 // Down a branch, with S(γ) = Σ c·ā(r)[owner]·ℓ(r-1)[other] over the splits γ
-// is a part of: ā(r-1) = φ_r ā(r) + ψ_r S.  A term is formed as (c·ℓ)·ā: c·ℓ is
-// the owner's value over γ's to a factor, while c and ā can each be near 2^100
-// in the FP32 form and c·ā pass its range.  Each split is seen by both its
+// is a part of: ā(r-1) = φ_r ā(r) + ψ_r S.  Each split is seen by both its
 // parts, so d/dψ_r = ½ Σ_γ ℓ(r-1)[γ] S(γ); d/dφ_r = Σ_γ ā(r)[γ] ℓ(r-1)[γ].
 // φ_r and ψ_r are functions of the branch's α, β and ε of row 0 alone
 // (src/model.jl:182-191): with den_r = 1 - β ε_{r-1}, φ_r = (1-α)(1-β)/den_r²
@@ -1480,7 +1478,7 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
               v[j] = T.V[o[j] >> 16];
             }
 #pragma unroll
-            for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(c[j] * v[j], a[j], t) : t;
+            for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(c[j] * a[j], v[j], t) : t;
           }
           t = slot_sum(t, pos, slot_steps(pos));
           if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : cA * t;
@@ -1505,10 +1503,10 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
 #pragma unroll
           for (int j = 0; j < kRecs; ++j) {
             const uint32_t y = o[j] >> 16;
-            const Real a = T.A[o[j] & 0xffffu];
-            tv = fma(c[j] * T.V[y], a, tv);
-            tf = fma(c[j] * T.F[y], a, tf);
-            tg = fma(c[j] * T.G[y], a, tg);
+            const Real x = c[j] * T.A[o[j] & 0xffffu];
+            tv = fma(x, T.V[y], tv);
+            tf = fma(x, T.F[y], tf);
+            tg = fma(x, T.G[y], tg);
           }
         }
         const int st = slot_steps(pos);
@@ -1732,7 +1730,7 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
         const uint32_t own = ent_ops[k] & 0xffffu, y = ent_ops[k] >> 16;
         Real c = (Real)ent_p[k];
         if (Scaled) c = coef_of(c, Ei, eit_at(y), eit_at(own));
-        fn(c, curA[own], y);
+        fn(c * curA[own], y);
       }
     };
     // one row of an item: its share of the sums, then ā(r-1); vn = ℓ(r-2)
@@ -1816,7 +1814,7 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
             for (int c = 0; c < NC_; ++c) {
               S_[c] = 0;
 #pragma unroll
-              for (int j = 0; j < KM; ++j) S_[c] = fma(q[c].c[j] * v_[c][j], a_[c][j], S_[c]);
+              for (int j = 0; j < KM; ++j) S_[c] = fma(q[c].c[j] * a_[c][j], v_[c][j], S_[c]);
             }
             if (steps > 0) {
 #pragma unroll
@@ -1842,8 +1840,8 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
           Real t = 0;
           const SliceRowB<Real> w = slice_b<Real>(pack, M.tab_rows, x.tab + (uint32_t)min(r, (int)x.R - 1));
 #pragma unroll
-          for (int j = 0; j < kRecs; ++j) t = fma(x.c[j] * curV[x.ops[j] >> 16], curA[x.ops[j] & 0xffffu], t);
-          rest(x, [&](Real c, Real a, uint32_t y) WHALE_INLINE { t = fma(c * curV[y], a, t); });
+          for (int j = 0; j < kRecs; ++j) t = fma(x.c[j] * curA[x.ops[j] & 0xffffu], curV[x.ops[j] >> 16], t);
+          rest(x, [&](Real c, uint32_t y) WHALE_INLINE { t = fma(c, curV[y], t); });
           t = slot_sum(t, x.pos, slot_steps(x.pos));
           finish(x, r, t, w, row_at(x, r - 2));
           if (!held) {
@@ -1881,13 +1879,13 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
       Real SF = 0, SG = 0;
 #pragma unroll
       for (int j = 0; j < kRecs; ++j) {
-        const Real a = curA[x.ops[j] & 0xffffu];
-        SF = fma(x.c[j] * bG[x.ops[j] >> 16], a, SF);
-        SG = fma(x.c[j] * bF[x.ops[j] >> 16], a, SG);
+        const Real c = x.c[j] * curA[x.ops[j] & 0xffffu];
+        SF = fma(c, bG[x.ops[j] >> 16], SF);
+        SG = fma(c, bF[x.ops[j] >> 16], SG);
       }
-      rest(x, [&](Real c, Real a, uint32_t y) WHALE_INLINE {
-        SF = fma(c * bG[y], a, SF);
-        SG = fma(c * bF[y], a, SG);
+      rest(x, [&](Real c, uint32_t y) WHALE_INLINE {
+        SF = fma(c, bG[y], SF);
+        SG = fma(c, bF[y], SG);
       });
       const int st = slot_steps(x.pos);
       SF = slot_sum(SF, x.pos, st);

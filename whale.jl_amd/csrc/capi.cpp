@@ -239,6 +239,9 @@ struct whale_batch {
     LaunchCfg cfg[2];  // forward, backward
   };
   std::vector<Group> groups[3];
+  // the same for a mixture of mix_k components (0: not planned since the classes were)
+  std::vector<Group> mix_groups[3];
+  int mix_k[3] = {0, 0, 0};
   LaunchCfg cfg_fb[2];             // FP64 pass over families the FP32 form could not represent
   int last_mode = -1;
   int last_launch = WHALE_LAUNCH_BATCHED;
@@ -946,9 +949,9 @@ bool fits_lds(const whale_batch* b, const FamDev& d) {
 // 1760); 777 families of 50 taxa, scaled FP64, 3350 -> 2200 us (kFill 1: 3140).
 // Past kFill the idle waves cost more than the launches: 5000 families, 2.5
 // times what the GPU holds, 3160 us apart, 3690 in two launches.
-void plan_groups(whale_batch* b, int mode) {
+// `comps`: that many components of a mixture run in every launch.
+void plan_groups(const whale_batch* b, int mode, int comps, std::vector<whale_batch::Group>& out) {
   const whale_model* m = b->model;
-  std::vector<whale_batch::Group>& out = b->groups[mode];
   out.clear();
   const uint32_t* ord = b->order_host.data();
   for (int j = 0; j < whale_batch::kClasses; ++j) {
@@ -965,7 +968,7 @@ void plan_groups(whale_batch* b, int mode) {
   // waves and LDS of a launch's families
   auto load = [&](const whale_batch::Group& g, double* w, double* l) {
     for (int d = 0; d < 2; ++d) {
-      const double n = (double)(g.hi - g.lo);
+      const double n = (double)comps * (g.hi - g.lo);
       w[d] += n * g.cfg[d].team;
       l[d] += n * (double)g.cfg[d].lds() / g.cfg[d].fpw;
     }
@@ -1031,7 +1034,10 @@ int plan_batch_launches(whale_batch* b) {
         if (!plan_families(b, dir == 0, mode, b->order_host.data() + lo, hi - lo, hi - lo, true, &b->cfg[mode][dir][k]))
           return fail(WHALE_EINVAL, "a family's largest stage does not fit the LDS of one compute unit");
       }
-  for (int mode = 0; mode < 3; ++mode) plan_groups(b, mode);
+  for (int mode = 0; mode < 3; ++mode) {
+    plan_groups(b, mode, 1, b->groups[mode]);
+    b->mix_k[mode] = 0;
+  }
   for (int dir = 0; dir < 2; ++dir)
     if (!plan_families(b, dir == 0, WHALE_FP64_SCALED, b->order_host.data(), b->order_host.size(),
                        (uint64_t)m->ctx->n_cu, false, &b->cfg_fb[dir]))
@@ -1902,29 +1908,27 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
   // one direction: every size class as one launch over all components on the
   // three streams, the families routed to FP64 as one launch beside them, and
   // the FP64 pass over the families each component's FP32 pass flagged
-  const int* kOrder = kLayoutOrder[b->tune.layout];
-  const int* kLane = kLayoutLane[b->tune.layout];
+  if (b->mix_k[mode] != K) {
+    plan_groups(b, mode, K, b->mix_groups[mode]);
+    b->mix_k[mode] = K;
+  }
+  const std::vector<whale_batch::Group>& groups = b->mix_groups[mode];
   auto direction = [&](int dir) -> int {
     constexpr int kLanes = 3;
     hipStream_t lanes[kLanes] = {st, c->side, c->side3};
     bool used[kLanes] = {};
-    for (int k = 0; k < whale_batch::kClasses; ++k)
-      if (b->cls_hi[k] > b->cls_lo[k]) used[kLane[k]] = true;
+    for (const auto& g : groups) used[g.lane] = true;
     const bool routed = b->route_lo < nf;
     HIPCHK(hipEventRecord(c->fork[3 * dir], st));
     for (int l = 1; l < kLanes; ++l)
       if (used[l]) HIPCHK(hipStreamWaitEvent(lanes[l], c->fork[3 * dir], 0));
     if (routed) HIPCHK(hipStreamWaitEvent(c->side2, c->fork[3 * dir], 0));
-    for (int q = 0; q < whale_batch::kClasses; ++q) {
-      const int k = kOrder[q];
-      if (b->cls_hi[k] == b->cls_lo[k]) continue;
-      hipStream_t sk = lanes[kLane[k]];
+    for (const auto& g : groups) {
       if (dir == 0)
-        HIPCHK(launch_forward(mode, store_all, b->cfg[mode][0][k], sk, B, M0, Wj[0], -1, b->cls_lo[k], b->cls_hi[k],
-                              nullptr, at(kF + k), K));
+        HIPCHK(launch_forward(mode, store_all, g.cfg[0], lanes[g.lane], B, M0, Wj[0], -1, g.lo, g.hi, nullptr,
+                              at(kF + g.cls), K));
       else
-        HIPCHK(launch_backward(mode, b->cfg[mode][1][k], sk, B, M0, Wj[0], -1, b->cls_lo[k], b->cls_hi[k], nullptr,
-                               at(kB + k), K));
+        HIPCHK(launch_backward(mode, g.cfg[1], lanes[g.lane], B, M0, Wj[0], -1, g.lo, g.hi, nullptr, at(kB + g.cls), K));
     }
     if (routed) {
       const int rmode = fp32 ? WHALE_FP64_SCALED : mode;

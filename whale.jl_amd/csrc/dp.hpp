@@ -1478,23 +1478,25 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
               v[j] = T.V[o[j] >> 16];
             }
 #pragma unroll
-            for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(c[j] * a[j], v[j], t) : t;
+            for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(cA * a[j] * c[j], v[j], t) : t;
           }
           t = slot_sum(t, pos, slot_steps(pos));
-          if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : cA * t;
+          if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : t;
         }
         tsync<Team, Gws>();
       }
       // With every ā known, all slots at once: with SF = Σ c·ā(owner)·G(other)
       // and SG likewise with F, ī of the tops is cB(ā ε_g + SF), cB(ā ε_f + SG);
-      // and the sums of d/dA, d/dB and the root children's ε.
+      // and the sums of d/dA, d/dB and the root children's ε.  The sums take
+      // the coefficient with the other part's value first: c·ā passes FP32's
+      // range where c·ā·ℓ does not.
 #pragma unroll 1
       for (uint32_t k0 = wv * kChunk; k0 < ns; k0 += nt) {
         const uint32_t k = k0 + lane;
         uint32_t z, r0, cnt;
         slot_of(k < ns ? k : 0u, k < ns, z, r0, cnt);
         const uint32_t i = z & 0xffffu, pos = (z >> 16) & 0xfu;
-        Real tv = 0, tf = 0, tg = 0;
+        Real tv = 0, tf = 0, tg = 0, tb = 0;
 #pragma unroll 1
         for (uint32_t j0 = 0; __any(j0 < cnt); j0 += kRecs) {
           uint32_t o[kRecs];
@@ -1503,22 +1505,24 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
 #pragma unroll
           for (int j = 0; j < kRecs; ++j) {
             const uint32_t y = o[j] >> 16;
-            const Real x = c[j] * T.A[o[j] & 0xffffu];
-            tv = fma(x, T.V[y], tv);
+            const Real a = T.A[o[j] & 0xffffu], g = T.G[y], x = a * c[j];
+            tv = fma(c[j] * T.V[y], a, tv);
+            tb = fma(c[j] * g, a, tb);
             tf = fma(x, T.F[y], tf);
-            tg = fma(x, T.G[y], tg);
+            tg = fma(x, g, tg);
           }
         }
         const int st = slot_steps(pos);
         tv = slot_sum(tv, pos, st);
         tf = slot_sum(tf, pos, st);
         tg = slot_sum(tg, pos, st);
+        tb = slot_sum(tb, pos, st);
         if (z & kSlotLead) {
           const Real a = T.A[i], v = T.V[i], vf = T.F[i], vg = T.G[i];
           ibar[sg.ibar + i] = cB * (a * eg + tg);
           ibar[sg.ibar + n + i] = cB * (a * ef + tf);
           sA += 0.5 * ((double)v * tv);
-          sB += (double)vf * tg + (double)a * ((double)vf * eg + (double)vg * ef);
+          sB += (double)vf * tb + (double)a * ((double)vf * eg + (double)vg * ef);
           sF += (double)a * vf;
           sG += (double)a * vg;
         }

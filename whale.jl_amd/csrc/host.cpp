@@ -539,14 +539,14 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
       }
     return true;
   };
-  // slots of the items [lo, hi) of the stage, in one direction
-  auto emit_slots = [&](const StageDev& sd, uint32_t lo, uint32_t hi, bool fwd, uint32_t offset) -> bool {
+  // slots of some of the stage's items, in one direction
+  auto emit_slots = [&](const StageDev& sd, const std::vector<uint32_t>& items, bool fwd, uint32_t offset) -> bool {
     const std::vector<uint32_t>& off = fwd ? r0 : e0;
     std::vector<uint32_t>&s4 = fwd ? F.fs4 : F.bs4, &s2 = fwd ? F.fs2 : F.bs2;
-    cnt.resize(hi - lo);
-    for (uint32_t i = lo; i < hi; ++i) {
-      cnt[i - lo] = off[i + 1] - off[i];
-      if (cnt[i - lo] > kSlotLanes * 0xffffu) { F.err = "clade with too many splits"; return false; }
+    cnt.resize(items.size());
+    for (size_t k = 0; k < items.size(); ++k) {
+      cnt[k] = off[items[k] + 1] - off[items[k]];
+      if (cnt[k] > kSlotLanes * 0xffffu) { F.err = "clade with too many splits"; return false; }
     }
     for (const auto& [k, pos] : deal_slots(cnt, offset)) {
       if (k < 0) {
@@ -554,7 +554,7 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
         s2.insert(s2.end(), {0u, 0u});
         continue;
       }
-      const uint32_t i = lo + (uint32_t)k, terms = cnt[k];
+      const uint32_t i = items[(size_t)k], terms = cnt[k];
       const uint32_t u = slot_lanes(terms);
       const uint32_t a = (uint32_t)((uint64_t)terms * pos / u), b = (uint32_t)((uint64_t)terms * (pos + 1) / u);
       const uint32_t si = F.it_seg[sd.item0 + i], gid = F.it_gid[sd.item0 + i];
@@ -585,13 +585,16 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
     }
     return true;
   };
+  std::vector<uint32_t> all;
   for (auto& st : stages) {
     StageDev sd{};
     if (!emit_items(st, sd)) return;
     if (sd.n_segs > 0xffff) { F.err = "stage with more than 65535 segments"; return; }
     sd.fs0 = (uint32_t)(F.fs4.size() / 4);
     sd.bs0 = (uint32_t)(F.bs4.size() / 4);
-    if (!emit_slots(sd, 0, sd.n_items, true, 0) || !emit_slots(sd, 0, sd.n_items, false, 0)) return;
+    all.resize(sd.n_items);
+    std::iota(all.begin(), all.end(), 0u);
+    if (!emit_slots(sd, all, true, 0) || !emit_slots(sd, all, false, 0)) return;
     sd.n_fs = (uint32_t)(F.fs4.size() / 4) - sd.fs0;
     sd.n_bs = (uint32_t)(F.bs4.size() / 4) - sd.bs0;
     F.max_items = std::max(F.max_items, sd.n_items);
@@ -604,29 +607,25 @@ void plan_family(const ModelHost& m, int32_t nc, const int32_t* csize, const int
     const size_t rec_before = F.rec_ops.size();
     if (!emit_items({m.root}, sd)) return;
     F.root_recs = (uint32_t)(F.rec_ops.size() - rec_before);
-    // root levels: runs of clades in size order of which none is a part of
-    // another, so a level reads only finished parts (and, in the reverse
-    // sweep, only finished owners).  Clades of one size never are; a run goes
-    // on past a size until a clade has a part inside it.
-    std::vector<uint32_t> lvl{0};
-    for (int c = 1, start = 0; c < nc; ++c) {
-      int32_t dep = -1;
-      for (int64_t k = soff[c]; k < soff[c + 1]; ++k) dep = std::max(dep, std::max(g1[k], g2[k]));
-      if (dep >= start) {
-        lvl.push_back((uint32_t)c);
-        start = c;
-      }
+    // Root levels by depth: a clade's level is one past the highest level of
+    // its splits' parts, so a level reads only finished parts and, in the
+    // reverse sweep, only finished owners.  (Runs of clades in size order of
+    // which none is a part of another: 21 to 26 levels for the families of 25
+    // genes at which depth gives 17 to 22, 116 against 44 for 240 genes.)
+    std::vector<uint32_t> depth(nc, 0);
+    std::vector<std::vector<uint32_t>> lvl(1);
+    for (int c = 0; c < nc; ++c) {
+      for (int64_t k = soff[c]; k < soff[c + 1]; ++k) depth[c] = std::max({depth[c], depth[g1[k]] + 1, depth[g2[k]] + 1});
+      if (depth[c] >= lvl.size()) lvl.resize(depth[c] + 1);
+      lvl[depth[c]].push_back((uint32_t)c);
     }
-    lvl.push_back((uint32_t)nc);
     F.root_fs = (uint32_t)(F.fs4.size() / 4);
     F.root_bs = (uint32_t)(F.bs4.size() / 4);
-    for (size_t L = 0; L < lvl.size(); ++L) {
+    for (size_t L = 0; L <= lvl.size(); ++L) {
       F.lvl_f.push_back((uint32_t)(F.fs4.size() / 4) - F.root_fs);
       F.lvl_b.push_back((uint32_t)(F.bs4.size() / 4) - F.root_bs);
-      if (L + 1 == lvl.size()) break;
-      if (!emit_slots(sd, lvl[L], lvl[L + 1], true, F.lvl_f.back()) ||
-          !emit_slots(sd, lvl[L], lvl[L + 1], false, F.lvl_b.back()))
-        return;
+      if (L == lvl.size()) break;
+      if (!emit_slots(sd, lvl[L], true, F.lvl_f.back()) || !emit_slots(sd, lvl[L], false, F.lvl_b.back())) return;
     }
   }
   // workload counts (the reference's cell and split-term counts)

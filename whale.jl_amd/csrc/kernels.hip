@@ -901,19 +901,35 @@ hipError_t launch_bt_pack(hipStream_t st, uint64_t walks, const int32_t* counts,
 
 // ---------------------------------------------------------------------------
 // k_det_sum: the batch's gradient accumulators as the sum of the per-family
-// slots in family order (one lane per accumulator), so that the result does
-// not depend on which workgroup evaluated which family, or when.
+// slots in an order that depends on the number of families alone, so that the
+// result does not depend on which workgroup evaluated which family, or when.
+// A workgroup sums 16 accumulators (a 128-byte line of every slot), 64 lanes
+// each; lane r takes families r, r + 64, …, and the lanes' sums are added
+// pairwise.  One lane an accumulator is a chain of n_fam loads: 190 us for 777
+// families of 50 taxa.
 // ---------------------------------------------------------------------------
-__global__ void k_det_sum(const double* slots, uint32_t n_fam, int ncol, double* out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= ncol) return;
-  double s = 0.0;
-  for (uint32_t f = 0; f < n_fam; ++f) s += slots[(size_t)f * ncol + j];
-  out[j] = s;
+constexpr int kDetCols = 16, kDetLanes = 64;
+__global__ __launch_bounds__(kDetCols * kDetLanes) void k_det_sum(const double* slots, uint32_t n_fam, int ncol,
+                                                                  double* out) {
+  __shared__ double s[kDetLanes][kDetCols];
+  const int c = threadIdx.x % kDetCols, r = threadIdx.x / kDetCols;
+  const int j = blockIdx.x * kDetCols + c;
+  double t = 0.0;
+  if (j < ncol) {
+#pragma unroll 8
+    for (uint32_t f = (uint32_t)r; f < n_fam; f += kDetLanes) t += slots[(size_t)f * ncol + j];
+  }
+  s[r][c] = t;
+  for (int w = kDetLanes / 2; w > 0; w >>= 1) {
+    __syncthreads();
+    if (r < w) s[r][c] += s[r + w][c];
+  }
+  if (r == 0 && j < ncol) out[j] = s[0][c];
 }
 
 hipError_t launch_det_sum(hipStream_t st, const double* slots, uint32_t n_fam, int ncol, double* out) {
-  hipLaunchKernelGGL(k_det_sum, dim3((ncol + 255) / 256), dim3(256), 0, st, slots, n_fam, ncol, out);
+  hipLaunchKernelGGL(k_det_sum, dim3((ncol + kDetCols - 1) / kDetCols), dim3(kDetCols * kDetLanes), 0, st, slots, n_fam,
+                     ncol, out);
   return hipGetLastError();
 }
 

@@ -26,8 +26,8 @@
 //            one pass; chunks are filled longest items first, so the lanes of
 //            a chunk have similar term counts.
 //   root     the last stage of every family: all clades, one row, processed
-//            in clade-size levels (the root term uses the root's own smaller
-//            clades, src/core.jl:151-158); its slots are listed level by
+//            in levels (the root term uses the root's own smaller clades,
+//            src/core.jl:151-158); its slots are listed level by
 //            level, an item's lanes within 16 slots from a multiple of 16.
 #pragma once
 #include <stdint.h>

@@ -138,7 +138,7 @@ struct whale_ctx {
 struct whale_model {
   whale_ctx* ctx = nullptr;
   ModelHost h;
-  DBuf nodes, eps, phi, psi, pack64, pack32, dnode, par, hlv, hnd, dlv, dnd, ebar, out;
+  DBuf nodes, eps, phi, psi, pack64, pack32, dnode, par, hlv, hnd, dlv, dnd, rown, twork, ebar;
   int n_hlevels = 0, n_dlevels = 0;
   bool has_params = false;
   std::vector<double> host_par;
@@ -510,6 +510,10 @@ int whale_model_create(whale_ctx* ctx, int32_t n, const int32_t* parent, const i
   HIPCHK(upload(m->hnd, hnd, st));
   HIPCHK(upload(m->dlv, dlv, st));
   HIPCHK(upload(m->dnd, dnd, st));
+  std::vector<int32_t> rown;  // every table row's node
+  for (int e = 0; e < n; ++e) rown.insert(rown.end(), (size_t)h.nodes[e].R, e);
+  HIPCHK(upload(m->rown, rown, st));
+  if (const size_t tw = tables_work_bytes(n, h.tab_rows); tw > kTabLds || tw > ctx->lds_wg) HIPCHK(m->twork.alloc(tw));
   HIPCHK(m->eps.alloc(sizeof(double) * h.tab_rows));
   HIPCHK(m->phi.alloc(sizeof(double) * h.tab_rows));
   HIPCHK(m->psi.alloc(sizeof(double) * h.tab_rows));
@@ -517,8 +521,7 @@ int whale_model_create(whale_ctx* ctx, int32_t n, const int32_t* parent, const i
   HIPCHK(m->pack32.alloc(sizeof(float) * 7 * h.tab_rows));
   HIPCHK(m->dnode.alloc(sizeof(double) * kDnode * n));
   HIPCHK(m->par.alloc(sizeof(double) * (3 * n + nwgd + 1)));
-  HIPCHK(m->ebar.alloc(sizeof(double) * n));
-  HIPCHK(m->out.alloc(sizeof(double) * (2 + 2 * n + nwgd)));
+  HIPCHK(m->ebar.alloc(tail_work_bytes(n)));
   *out = m.release();
   return WHALE_OK;
 }
@@ -550,7 +553,7 @@ int whale_model_set_params(whale_model* m, const double* lambda, const double* m
   HIPCHK(hipMemcpyAsync(m->par.p, hp.data(), hp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIPCHK(launch_tables(c->stream, m->dev(), m->eps.as<double>(), m->phi.as<double>(), m->psi.as<double>(),
                        m->pack64.as<double>(), m->pack32.as<float>(), m->dnode.as<double>(), m->hlv.as<int32_t>(), m->hnd.as<int32_t>(),
-                       m->n_hlevels));
+                       m->n_hlevels, m->rown.as<int32_t>(), m->twork.as<double>()));
   if (c->timing) HIPCHK(hipEventRecord(c->ev[1], c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   if (c->timing) {
@@ -1256,14 +1259,9 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   W.seed = b->seeded && grad ? b->seed.as<double>() : nullptr;
   const AccLayout AL(m->h.n, m->h.n_wgd);
   if (timed) HIPCHK(hipEventRecord(c->ev[1], st));
-  HIPCHK(launch_fill_u32(st, W.ticket, 0u, kTickets));
-  if (grad) HIPCHK(launch_fill_f64(st, W.acc, 0.0, AL.n));
   const uint32_t nf = b->n_fam;
   const bool fp32 = mode == WHALE_FP32_SCALED;
-  if (fp32) {
-    HIPCHK(launch_fill_u32(st, W.flag, 0u, (int)nf));
-    HIPCHK(launch_fill_u32(st, W.fb, 0u, 1));
-  }
+  HIPCHK(launch_reset(st, W.ticket, kTickets, W.acc, grad ? AL.n : 0, W.flag, fp32 ? (int)nf : 0, W.fb));
   // families the FP32 pass could not represent, recomputed in FP64 with per-clade exponents
   BatchDev Bfb = B;
   Bfb.order = W.fb + 1;
@@ -1455,16 +1453,14 @@ int enqueue(whale_batch* b, int mode, int32_t launch, bool grad, bool store_all,
   if (timed) HIPCHK(hipEventRecord(c->ev[3], st));
   }
   if (W.acc_fam) HIPCHK(launch_det_sum(st, W.acc_fam, nf, AL.n, W.acc));
-  double* out = ws_out ? ws_out : m->out.as<double>();
-  HIPCHK(launch_tail(st, M, W.fam_ll, nf, W.acc, m->ebar.as<double>(),
-                     m->dlv.as<int32_t>(), m->dnd.as<int32_t>(), m->n_dlevels, m->h.cond, grad ? 1 : 0, out,
-                     W.seed ? W.seed + nf : nullptr));
-  if (timed) HIPCHK(hipEventRecord(c->ev[4], st));
-  if (ws) return WHALE_OK;
+  // the results go to the caller's device buffer, or from the kernel straight
+  // to the batch's pinned ones (three copies took 14 us of a small evaluation)
   const int n = m->h.n, nw = m->h.n_wgd;
-  HIPCHK(hipMemcpyAsync(b->pin_out, out, sizeof(double) * (grad ? 2 + 2 * n + nw : 1), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(b->pin_fam, W.fam_ll, sizeof(double) * nf, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(&b->pin_out[2 + 2 * n + nw], W.fb, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+  HIPCHK(launch_tail(st, M, W.fam_ll, nf, W.acc, m->ebar.as<double>(), m->dlv.as<int32_t>(), m->dnd.as<int32_t>(),
+                     m->n_dlevels, m->h.cond, grad ? 1 : 0, ws ? ws_out : b->pin_out, W.seed ? W.seed + nf : nullptr,
+                     ws ? nullptr : b->pin_fam, fp32 ? W.fb : nullptr,
+                     ws ? nullptr : reinterpret_cast<uint32_t*>(&b->pin_out[2 + 2 * n + nw])));
+  if (timed) HIPCHK(hipEventRecord(c->ev[4], st));
   return WHALE_OK;
 }
 
@@ -1898,12 +1894,8 @@ int whale_mixture_eval(whale_batch* b, whale_model* const* comps, int32_t K, con
   const ModelDev M0 = m0->dev();
   const bool store_all = grad;
   for (int j = 0; j < K; ++j) {
-    HIPCHK(launch_fill_u32(st, Wj[j].ticket, 0u, kTickets));
-    if (grad) HIPCHK(launch_fill_f64(st, Wj[j].acc, 0.0, AL.n));
-    if (fp32) {
-      HIPCHK(launch_fill_u32(st, Wj[j].flag, 0u, (int)nf));
-      HIPCHK(launch_fill_u32(st, Wj[j].fb, 0u, 1));
-    }
+    HIPCHK(launch_reset(st, Wj[j].ticket, kTickets, Wj[j].acc, grad ? AL.n : 0, Wj[j].flag, fp32 ? (int)nf : 0,
+                        Wj[j].fb));
   }
   // one direction: every size class as one launch over all components on the
   // three streams, the families routed to FP64 as one launch beside them, and

@@ -221,15 +221,22 @@ hipError_t launch_fused(int mode, const LaunchCfg& C, hipStream_t st, const Batc
                         const WorkRaw& W, uint32_t fam_begin, uint32_t fam_end, const uint32_t* fam_count, int grad,
                         const FusedSlots& SL);
 hipError_t launch_tables(hipStream_t st, const ModelDev& M, double* eps, double* phi, double* psi, double* pack64,
-                         float* pack32, double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels);
+                         float* pack32, double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels,
+                         const int32_t* row_node, double* work);
+// the workspace of launch_tables: in LDS up to kTabLds (`work` null), else `work`
+constexpr size_t kTabLds = 128 * 1024;
+size_t tables_work_bytes(int n, int rows);
 // n_eff (null: n_fam) holds the family count the conditioning term's
 // derivative is scaled by (Σ of the reverse sweep's family weights)
 hipError_t launch_tail(hipStream_t st, const ModelDev& M, const double* fam_ll, uint32_t n_fam, const double* acc,
-                       double* ebar, const int32_t* dlevels, const int32_t* dnodes, int n_dlevels, int cond, int with_grad, double* out,
-                       const double* n_eff = nullptr);
+                       double* work, const int32_t* dlevels, const int32_t* dnodes, int n_dlevels, int cond,
+                       int with_grad, double* out, const double* n_eff = nullptr, double* host_fam = nullptr,
+                       const uint32_t* fb = nullptr, uint32_t* host_fb = nullptr);
+size_t tail_work_bytes(int n);  // `work` of launch_tail
+hipError_t launch_reset(hipStream_t st, uint32_t* ticket, int n_ticket, double* acc, int n_acc, uint32_t* flag,
+                        int n_flag, uint32_t* fb);
 hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, int n);
 hipError_t launch_det_sum(hipStream_t st, const double* slots, uint32_t n_fam, int ncol, double* out);
-hipError_t launch_fill_f64(hipStream_t st, double* p, double v, size_t n);
 
 // What the backtracking sampler reads: the stored ℓ (FP32 or FP64 values,
 // plus the FP64 region of families an FP32 call evaluated in FP64), the

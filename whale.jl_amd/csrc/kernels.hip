@@ -26,9 +26,16 @@ namespace whale {
 // form.  The tops of the branches go level by level (a node's bottom value is
 // a function of its children's tops), one lane per node; then every row of
 // every branch is independent: ε(r−1) in closed form, then the last step and
-// the row's φ and ψ as the slice recursion writes them.  Last, one lane per
-// node runs ∂ε_r/∂(α, β, ε_0) up its rows for the reverse sweep's tables:
-// with den_r = 1 - β ε_{r-1}, D_k(r) = -(∂den_r/∂k)/den_r.
+// the row's φ and ψ as the slice recursion writes them.  Last,
+// ∂ε_r/∂(α, β, ε_0) for the reverse sweep's tables: with den_r = 1 - β ε_{r-1},
+// D_k(r) = -(∂den_r/∂k)/den_r.
+// The time is that of its chains: the levels of the tree, and the rows of the
+// longest branch.  So a level's step holds a few FP64 operations and divides
+// only (the functions and the loads come before), and the derivatives' chain
+// one multiply-add a row, its coefficients formed by all lanes at once in LDS.
+// Measured, with α, β and the functions within each step before -> now: 9 taxa
+// and 140 rows 23 -> 11 us, 58 taxa and slices of 0.01 53 -> 24 us, 50 taxa and
+// 1488 rows 60 -> 26 us.
 // ---------------------------------------------------------------------------
 struct SliceAB {
   double a, b, dal, dam, dbl, dbm;
@@ -68,25 +75,41 @@ __device__ inline SliceAB slice_ab(double l, double u, double t) {
 // keeps ε_k = ρ + (excess) free of cancellation.  κ^k and S go through
 // log1p/expm1 (κ is near 1 for short slices) and are scaled by κ^−k when
 // κ > 1.  Accurate to a few ulp, where k dependent steps drift by k ulp.
-__device__ inline double eps_after(double a, double b, int k, double e0) {
+// What does not depend on e0 comes first, so that the chain from the leaves to
+// the root holds none of the functions.
+// δ = κ − 1 of the α and β as they are stored.  Not to be fused with the
+// product β is formed by: near λ = μ the difference is all rounding, and S
+// needs the very δ that log κ was formed from.
+__device__ inline double slice_excess(double a, double b) {
+#pragma clang fp contract(off)
+  return (a - b) / (1.0 - a);
+}
+struct Powers {
+  double L, X, S;  // k·log κ; κ^±k and S (scaled by κ^−k), the sign that of −L
+};
+__device__ inline Powers slice_powers(double a, double b, double lg, int k) {
+  const double d = slice_excess(a, b);
+  Powers w{(double)k * lg, 1.0, (double)k};
+  if (d == 0.0) return w;
+  const double m = w.L <= 0.0 ? w.L : -w.L;
+  w.X = exp(m);
+  w.S = (w.L <= 0.0 ? expm1(m) : -expm1(m)) / d;
+  return w;
+}
+__device__ inline double eps_after(double a, double b, const Powers& w, int k, double e0) {
   if (k == 0 || e0 == 1.0) return e0;
   const double om = 1.0 - a;
   if (om == 0.0) return 1.0;
-  const double d = (a - b) / om;
+  const double d = slice_excess(a, b);
   if (a < b * e0) {
     const double rho = a / b;
-    const double W = exp((double)k * log1p(d)) * (e0 - rho) / (1.0 - e0);
+    const double W = (w.L <= 0.0 ? w.X : exp(w.L)) * (e0 - rho) / (1.0 - e0);
     return (rho + W) / (1.0 + W);
   }
   const double al = (a - b * e0) / om, be = b * (1.0 - e0) / om;
   if (d == 0.0) return (e0 + (double)k * al) / (1.0 + (double)k * be);
-  const double L = (double)k * log1p(d);
-  if (L <= 0.0) {
-    const double S = expm1(L) / d;
-    return (e0 + S * al) / (exp(L) + S * be);
-  }
-  const double SK = -expm1(-L) / d;  // S/κ^k
-  return (e0 * exp(-L) + SK * al) / (1.0 + SK * be);
+  if (w.L <= 0.0) return (e0 + w.S * al) / (w.X + w.S * be);
+  return (e0 * w.X + w.S * al) / (1.0 + w.S * be);
 }
 
 // one slice step from ε' = ep (the row's ε, φ, ψ)
@@ -99,123 +122,172 @@ __device__ inline void slice_step(double a, double b, double ep, double* en, dou
   *den_ = den;
 }
 
-__device__ inline double node_e0(const ModelDev& M, const NodeDev& d, int e) {
-  const double* p = M.par + 2 * M.n;
-  const double* q = M.par + 3 * M.n;
-  if (d.kind == WHALE_NODE_WGD) {
-    double ec = eps_top(M, d.child0);
-    double qq = q[d.wgd];
-    return qq * (ec * ec) + (1.0 - qq) * ec;
-  }
-  if (d.kind == WHALE_NODE_LEAF) return p[e];
-  return eps_top(M, d.child0) * eps_top(M, d.child1);
-}
+// The workspace of k_tables: per node α, β, log κ, the powers of its top and
+// its top ε; per row ε and the three coefficients of the derivatives' chain,
+// which their values replace.  In LDS where it fits.
+size_t tables_work_bytes(int n, int rows) { return 8 * (7 * (size_t)n + 4 * (size_t)rows); }
 
+template <bool InLds>
 __global__ __launch_bounds__(1024) void k_tables(ModelDev M, double* eps, double* phi, double* psi,
                                                     double* pack64, float* pack32, double* dnode,
-                                                    const int32_t* hlevels, const int32_t* hnodes, int n_levels) {
-  // row t of the packed tables: its φ, ψ, and χ, D_α, D_β, D_ε0
-  auto put_slice = [&](int t, double ph, double ps) {
-    const size_t n4 = 4 * (size_t)M.tab_rows;
-    pack64[4 * (size_t)t] = pack64[n4 + 2 * (size_t)t] = ph;
-    pack64[n4 + 2 * (size_t)t + 1] = ps;
-    pack32[4 * (size_t)t] = pack32[n4 + 2 * (size_t)t] = (float)ph;
-    pack32[n4 + 2 * (size_t)t + 1] = (float)ps;
-  };
-  auto put_den = [&](int t, double ch, double da, double db, double d0) {
-    const double v[4] = {ch, da, db, d0};
-    for (int j = 0; j < 4; ++j) {
-      const size_t i = j < 3 ? 4 * (size_t)t + 1 + j : 6 * (size_t)M.tab_rows + t;
-      pack64[i] = v[j];
-      pack32[i] = (float)v[j];
-    }
-  };
-  extern __shared__ int32_t s_tab[];  // first table row of each node, then tab_rows
+                                                    const int32_t* hlevels, const int32_t* hnodes, int n_levels,
+                                                    const int32_t* row_node, double* work) {
+  extern __shared__ __align__(16) double s_work[];
+  const int n = M.n, rows = M.tab_rows, t = threadIdx.x, nt = blockDim.x;
+  double* const A = InLds ? s_work : work;
+  double *const B = A + n, *const LG = B + n, *const PL = LG + n, *const PX = PL + n, *const PS = PX + n,
+                *const TOP = PS + n;
+  double *const EN = TOP + n, *const G = EN + rows, *const CA = G + rows, *const CB = CA + rows;
   const double* lam = M.par;
-  const double* mu = M.par + M.n;
-  for (int e = threadIdx.x; e < M.n; e += blockDim.x) s_tab[e] = M.node[e].tab;
-  if (threadIdx.x == 0) s_tab[M.n] = M.tab_rows;
-  // tops, children first
-  for (int L = 0; L < n_levels; ++L) {
-    for (int k = hlevels[L] + threadIdx.x; k < hlevels[L + 1]; k += blockDim.x) {
-      const int e = hnodes[k];
-      const NodeDev& d = M.node[e];
-      const int t0 = d.tab;
-      const double e0 = node_e0(M, d, e);
-      eps[t0] = e0;
-      phi[t0] = 1.0;
-      psi[t0] = 1.0;
-      put_slice(t0, 1.0, 1.0);
-      SliceAB s{0, 0, 0, 0, 0, 0};
-      if (d.R > 1) s = slice_ab(lam[e], mu[e], d.delta);
-      double* dn = dnode + (size_t)kDnode * e;
-      dn[0] = s.dal;
-      dn[1] = s.dam;
-      dn[2] = s.dbl;
-      dn[3] = s.dbm;
-      if (d.R > 1) {
-        double en, ph, ps, den;
-        slice_step(s.a, s.b, eps_after(s.a, s.b, d.R - 2, e0), &en, &ph, &ps, &den);
-        eps[t0 + d.R - 1] = en;
-      }
+  const double* mu = M.par + n;
+  const double* par_p = M.par + 2 * n;
+  const double* par_q = M.par + 3 * n;
+  // every node's slice map
+  for (int e = t; e < n; e += nt) {
+    const NodeDev& d = M.node[e];
+    SliceAB s{0, 0, 0, 0, 0, 0};
+    Powers w{0.0, 1.0, 0.0};
+    double lg = 0.0;
+    const bool br = d.R > 1;
+    if (br) {
+      s = slice_ab(lam[e], mu[e], d.delta);
+      lg = log1p(slice_excess(s.a, s.b));
+      w = slice_powers(s.a, s.b, lg, d.R - 2);
     }
-    __syncthreads();
+    A[e] = s.a;
+    B[e] = s.b;
+    LG[e] = lg;
+    PL[e] = w.L;
+    PX[e] = w.X;
+    PS[e] = w.S;
+    const double ia = 1.0 / (1.0 - s.a), ib = 1.0 / (1.0 - s.b);
+    // at α or β = 1 no lineage crosses the branch: φ = ψ = 0 and the sums these multiply are 0
+    const double v[7] = {s.dal, s.dam, s.dbl, s.dbm, br && isfinite(ia) ? ia : 0.0, br && isfinite(ib) ? ib : 0.0,
+                         br ? s.b : 0.0};
+#pragma unroll
+    for (int j = 0; j < 7; ++j) dnode[(size_t)kDnode * e + j] = v[j];
   }
-  // every row r ≥ 1 of every branch
-  for (int t = threadIdx.x; t < M.tab_rows; t += blockDim.x) {
-    int lo = 0, hi = M.n;  // the node e with s_tab[e] ≤ t < s_tab[e + 1]
+  // tops, children first: a lane keeps the entry of hnodes that is its own
+  const int me = t < n ? hnodes[t] : -1;
+  const NodeDev mine = M.node[me >= 0 ? me : 0];
+  int lv = -1;
+  if (me >= 0) {
+    int lo = 0, hi = n_levels;  // the level L with hlevels[L] ≤ t < hlevels[L + 1]
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
-      if (s_tab[mid] <= t) lo = mid;
+      if (hlevels[mid] <= t) lo = mid;
       else hi = mid;
     }
-    const int e = lo;
-    const int r = t - s_tab[e];
-    if (r == 0) continue;
+    lv = lo;
+  }
+  auto top = [&](int e, const NodeDev& d) {
+    double e0;
+    if (d.kind == WHALE_NODE_WGD) {
+      const double ec = TOP[d.child0], qq = par_q[d.wgd];
+      e0 = qq * (ec * ec) + (1.0 - qq) * ec;
+    } else if (d.kind == WHALE_NODE_LEAF) {
+      e0 = par_p[e];
+    } else {
+      e0 = TOP[d.child0] * TOP[d.child1];
+    }
+    EN[d.tab] = e0;
+    double en = e0;
+    if (d.R > 1) {
+      const double a = A[e], b = B[e];
+      double ph, ps, den;
+      slice_step(a, b, eps_after(a, b, Powers{PL[e], PX[e], PS[e]}, d.R - 2, e0), &en, &ph, &ps, &den);
+      EN[d.tab + d.R - 1] = en;
+    }
+    TOP[e] = en;
+  };
+  __syncthreads();
+  for (int L = 0; L < n_levels; ++L) {
+    if (lv == L) top(me, mine);
+    for (int k = t + nt; k < n; k += nt)  // trees of more nodes than lanes
+      if (k >= hlevels[L] && k < hlevels[L + 1]) top(hnodes[k], M.node[hnodes[k]]);
+    __syncthreads();
+  }
+  // every row: ε(r−1) in closed form, then the last step
+  auto put = [&](size_t i, double v) {
+    pack64[i] = v;
+    pack32[i] = (float)v;
+  };
+  const size_t n4 = 4 * (size_t)rows, n6 = 6 * (size_t)rows;
+  for (int i = t; i < rows; i += nt) {
+    const int e = row_node[i];
     const NodeDev& d = M.node[e];
-    const SliceAB s = slice_ab(lam[e], mu[e], d.delta);
-    const double a = s.a, b = s.b;
-    const double ep = eps_after(a, b, r - 1, eps[d.tab]);
-    double en, ph, ps, den;
-    slice_step(a, b, ep, &en, &ph, &ps, &den);
-    if (r == d.R - 1)
-      en = eps[t];  // the top, as the levels wrote it for the parent
-    else
-      eps[t] = en;
-    phi[t] = ph;
-    psi[t] = ps;
-    put_slice(t, ph, ps);
+    const int r = i - d.tab;
+    double en, ph = 1.0, ps = 1.0, den;
+    if (r == 0) {
+      en = EN[i];
+    } else {
+      const double a = A[e], b = B[e];
+      slice_step(a, b, eps_after(a, b, slice_powers(a, b, LG[e], r - 1), r - 1, EN[d.tab]), &en, &ph, &ps, &den);
+      if (r == d.R - 1) en = EN[i];  // the top, as the levels wrote it for the parent
+      else EN[i] = en;
+    }
+    eps[i] = en;
+    phi[i] = ph;
+    psi[i] = ps;
+    put(4 * (size_t)i, ph);
+    put(n4 + 2 * (size_t)i, ph);
+    put(n4 + 2 * (size_t)i + 1, ps);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < M.n; e += blockDim.x) {
+  // ∂ε_r/∂(α, β, ε_0) as a chain of z ← G z + c
+  for (int i = t; i < rows; i += nt) {
+    const int e = row_node[i];
+    if (i == M.node[e].tab) continue;
+    const double a = A[e], b = B[e], ep = EN[i - 1], en = EN[i];
+    const double id = 1.0 / (1.0 - b * ep);
+    G[i] = ((1.0 - a - b) + b * en) * id;
+    CA[i] = (1.0 - ep) * id;
+    CB[i] = ep * (en - 1.0) * id;
+  }
+  __syncthreads();
+  for (int e = t; e < n; e += nt) {
     const NodeDev& d = M.node[e];
-    double* dn = dnode + (size_t)kDnode * e;
-    put_den(d.tab, 0.0, 0.0, 0.0, 0.0);  // row 0 has no slice
-    double za = 0.0, zb = 0.0, z0 = 1.0;  // ∂ε_{r-1}/∂(α, β, ε_0)
-    dn[4] = dn[5] = dn[6] = 0.0;
-    if (d.R > 1) {
-      const SliceAB s = slice_ab(lam[e], mu[e], d.delta);
-      const double a = s.a, b = s.b;
-      const double ia = 1.0 / (1.0 - a), ib = 1.0 / (1.0 - b);
-      // at α or β = 1 no lineage crosses the branch: φ = ψ = 0 and the sums these multiply are 0
-      dn[4] = isfinite(ia) ? ia : 0.0;
-      dn[5] = isfinite(ib) ? ib : 0.0;
-      dn[6] = b;
-      double ep = eps[d.tab];
-      for (int r = 1; r < d.R; ++r) {
-        const double en = eps[d.tab + r];
-        const double den = 1.0 - b * ep, id = 1.0 / den;
-        put_den(d.tab + r, (1.0 - a) * (1.0 - b) / (den * den * den), b * za * id, (ep + b * zb) * id, b * z0 * id);
-        const double G2 = ((1.0 - a - b) + b * en) * id;
-        za = (1.0 - ep) * id + G2 * za;
-        zb = ep * (en - 1.0) * id + G2 * zb;
-        z0 = G2 * z0;
-        ep = en;
+    double za = 0.0, zb = 0.0, z0 = 1.0;
+    const int i1 = d.tab + d.R;
+    constexpr int U = 8;  // rows read at once, ahead of the chain
+    for (int i0 = d.tab + 1; i0 < i1; i0 += U) {
+      double g[U], ca[U], cb[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = min(i0 + u, i1 - 1);
+        g[u] = G[i], ca[u] = CA[i], cb[u] = CB[i];
       }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u < i1) {
+          G[i0 + u] = z0, CA[i0 + u] = za, CB[i0 + u] = zb;
+          za = ca[u] + g[u] * za;
+          zb = cb[u] + g[u] * zb;
+          z0 = g[u] * z0;
+        }
     }
+    double* dn = dnode + (size_t)kDnode * e;
+    const bool br = d.R > 1;
     dn[7] = z0;
-    dn[8] = za;
-    dn[9] = zb;
+    dn[8] = br ? za : 0.0;
+    dn[9] = br ? zb : 0.0;
+  }
+  __syncthreads();
+  for (int i = t; i < rows; i += nt) {
+    const int e = row_node[i];
+    double ch = 0.0, da = 0.0, db = 0.0, d0 = 0.0;  // row 0 has no slice
+    if (i != M.node[e].tab) {
+      const double a = A[e], b = B[e], ep = EN[i - 1];
+      const double den = 1.0 - b * ep, id = 1.0 / den;
+      ch = (1.0 - a) * (1.0 - b) / (den * den * den);
+      da = b * CA[i] * id;
+      db = (ep + b * CB[i]) * id;
+      d0 = b * G[i] * id;
+    }
+    put(4 * (size_t)i + 1, ch);
+    put(4 * (size_t)i + 2, da);
+    put(4 * (size_t)i + 3, db);
+    put(n6 + i, d0);
   }
 }
 
@@ -303,92 +375,136 @@ __global__ __launch_bounds__(1024) void k_mix(const MixComp* X, int K, const dou
 
 constexpr int kTailThreads = 1024;
 
-// k_tail: one workgroup.  Σℓ over the families, the conditioning term, and
-// the chain rule from the nodes' sums to ∂λ, ∂μ, ∂q, ∂η.  The adjoints of a
-// branch's ε of row 0, α and β are its own sums plus the adjoint of its top ε
-// times ∂ε_top/∂(ε_0, α, β) (k_tables); depth by depth, parents first, a
-// node's top adjoint takes its parent's row-0 one.
+// Sum over the workgroup, in every lane of it: lanes of a wave, then waves.
+__device__ inline double group_sum(double v, double* part) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int w = 0; w < kTailThreads / 64; ++w) s += part[w];
+  return s;
+}
+
+// The workspace of k_tail, per node: ε̄ of its top and what the chain from the
+// root needs of it; the levels of the tree.  In LDS where it fits.
+constexpr size_t kTailLds = 48 * 1024;
+size_t tail_work_bytes(int n) { return 8 * 4 * (size_t)n; }
+
+// k_tail.  The first workgroup forms Σℓ over the families, the conditioning
+// term, and the chain rule from the nodes' sums to ∂λ, ∂μ, ∂q, ∂η.  The
+// adjoints of a branch's ε of row 0, α and β are its own sums plus the adjoint
+// of its top ε times ∂ε_top/∂(ε_0, α, β) (k_tables); depth by depth, parents
+// first, a node's top adjoint takes its parent's row-0 one.  Only that chain
+// goes by depth, one multiply-add and two products a level on values loaded
+// before it; all else follows for every node at once.
+// Results may go to pinned host memory: `out`, and with `host_fam` every
+// family's ℓ and the count *fb of families recomputed in FP64.  The other
+// workgroups share the families' copy.
+// Measured, with the chain on global memory and a tree reduction of Σℓ before
+// -> now: 12 families of 9 taxa 13.5 -> 6.4 us, one of 58 taxa 16.7 -> 6.1 us,
+// 10,000 of 50 taxa 30 -> 13 us, the three copies to the host (14 us) included
+// in the latter figures.
+template <bool InLds>
 __global__ __launch_bounds__(kTailThreads) void k_tail(ModelDev M, const double* fam_ll, uint32_t n_fam,
-                                                       const double* acc_in, double* ebar, const int32_t* dlevels,
+                                                       const double* acc_in, double* work, const int32_t* dlevels,
                                                        const int32_t* dnodes, int n_dlevels, int cond, int with_grad,
-                                                       double* out, const double* n_eff) {
-  __shared__ double red[kTailThreads];
-  __shared__ double s_total, s_eta;
-  const int t = threadIdx.x;
-  const AccLayout AL(M.n, M.n_wgd);
+                                                       double* out, const double* n_eff, double* host_fam,
+                                                       const uint32_t* fb, uint32_t* host_fb) {
+  extern __shared__ __align__(16) double s_work[];
+  __shared__ double part[kTailThreads / 64];
+  __shared__ CondTerms s_ct;
+  const int t = threadIdx.x, n = M.n;
+  if (host_fam)
+    for (uint32_t i = blockIdx.x * blockDim.x + t; i < n_fam; i += gridDim.x * blockDim.x) host_fam[i] = fam_ll[i];
+  if (blockIdx.x > 0) return;
+  const AccLayout AL(n, M.n_wgd);
+  double *const EB = InLds ? s_work : work, *const SL = EB + n, *const E0 = SL + n, *const TOP = E0 + n;
+  // the last wave forms the conditioning term while the others load
+  if (t == kTailThreads - 1) s_ct = cond_terms(M, cond);
+  NodeDev mine{};
+  int me = -1, lv = -1;
+  if (with_grad) {
+    for (int e = t; e < n; e += blockDim.x) {
+      const double* dn = M.dnode + (size_t)kDnode * e;
+      EB[e] = acc_in[AL.eps + e];
+      SL[e] = dn[7];
+      E0[e] = acc_in[AL.e0 + e];
+      TOP[e] = eps_top(M, e);
+    }
+    if (t < n) {  // a lane's own entry of dnodes, in level lv
+      me = dnodes[t];
+      mine = M.node[me];
+      int lo = 0, hi = n_dlevels;
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (dlevels[mid] <= t) lo = mid;
+        else hi = mid;
+      }
+      lv = lo;
+    }
+  }
+  if (t == 0 && host_fb) *host_fb = fb ? *fb : 0u;
   // Σ ℓ_i
   double s = 0;
+#pragma unroll 4
   for (uint32_t i = t; i < n_fam; i += blockDim.x) s += fam_ll[i];
-  red[t] = s;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
-  }
-  const NodeDev& rn = M.node[M.root];
-  const double eta = M.par[3 * M.n + M.n_wgd];
-  const double er = eps_top(M, M.root);
-  const CondTerms CT = cond_terms(M, cond);
-  const double c = CT.c, dc_er = CT.dc_er, dc_ef = CT.dc_ef, dc_eg = CT.dc_eg, dc_eta = CT.dc_eta;
-  const double N = (double)n_fam;
+  s = group_sum(s, part);  // its barrier also shows s_ct and the arrays
+  const CondTerms CT = s_ct;
   if (t == 0) {
-    const double tot = red[0] - N * c;
-    s_total = isfinite(tot) ? tot : -INFINITY;
+    const double tot = s - (double)n_fam * CT.c;
+    out[0] = isfinite(tot) ? tot : -INFINITY;
   }
-  if (!with_grad) {
-    if (t == 0) out[0] = s_total;
-    return;
-  }
-  // ε̄ of every node's top row: DP contributions + conditioning + root A/B terms
-  for (int e = t; e < M.n; e += blockDim.x) ebar[e] = acc_in[AL.eps + e];
-  __syncthreads();
+  if (!with_grad) return;
   if (t == 0) {
+    // ε̄ of the top rows: conditioning and root A/B terms beside the DP's
+    const NodeDev& rn = M.node[M.root];
+    const double eta = M.par[3 * n + M.n_wgd];
+    const double er = TOP[M.root];
     const double A_ = acc_in[AL.rootA], B_ = acc_in[AL.rootB];
     const double xi = 1.0 - (1.0 - eta) * er;
     const double dA_deta = (-xi + (1.0 - eta) * er) / eta - (1.0 - eta) * xi / (eta * eta);
     const double dA_der = -(1.0 - eta) * (1.0 - eta) / eta;
     const double dB_deta = (1.0 - er) / (xi * xi) - 2.0 * eta * (1.0 - er) * er / (xi * xi * xi);
     const double dB_der = -eta / (xi * xi) + 2.0 * eta * (1.0 - er) * (1.0 - eta) / (xi * xi * xi);
-    const double Ng = n_eff ? *n_eff : N;  // the families' weight in the gradient
-    ebar[M.root] += A_ * dA_der + B_ * dB_der - Ng * dc_er;
-    ebar[rn.child0] += -Ng * dc_ef;
-    ebar[rn.child1] += -Ng * dc_eg;
-    s_eta = A_ * dA_deta + B_ * dB_deta - Ng * dc_eta;
+    const double Ng = n_eff ? *n_eff : (double)n_fam;  // the families' weight in the gradient
+    EB[M.root] += A_ * dA_der + B_ * dB_der - Ng * CT.dc_er;
+    EB[rn.child0] += -Ng * CT.dc_ef;
+    EB[rn.child1] += -Ng * CT.dc_eg;
+    out[1 + 2 * n + M.n_wgd] = A_ * dA_deta + B_ * dB_deta - Ng * CT.dc_eta;
   }
   __syncthreads();
-  double* dl = out + 1;
-  double* dm = out + 1 + M.n;
-  double* dq = out + 1 + 2 * M.n;
-  for (int w = t; w < M.n_wgd; w += blockDim.x) dq[w] = acc_in[AL.q + w];
-  __syncthreads();
-  // parents before children
-  for (int L = 0; L < n_dlevels; ++L) {
-    for (int k = dlevels[L] + t; k < dlevels[L + 1]; k += blockDim.x) {
-      const int e = dnodes[k];
-      const NodeDev& d = M.node[e];
-      const double gt = ebar[e];
-      const double* dn = M.dnode + (size_t)kDnode * e;
-      const double g = dn[7] * gt + acc_in[AL.e0 + e];  // ε̄ of row 0
-      const double ga = dn[8] * gt + acc_in[AL.da + e], gb = dn[9] * gt + acc_in[AL.db + e];
-      dl[e] = d.R > 1 ? ga * dn[0] + gb * dn[2] : 0.0;
-      dm[e] = d.R > 1 ? ga * dn[1] + gb * dn[3] : 0.0;
-      // row 0 of ε: product of the children's tops, or the WGD retention map
-      if (d.kind == WHALE_NODE_WGD) {
-        const double ec = eps_top(M, d.child0);
-        const double qq = M.par[3 * M.n + d.wgd];
-        ebar[d.child0] += g * (2.0 * qq * ec + (1.0 - qq));
-        dq[d.wgd] += g * (ec * ec - ec);
-      } else if (d.kind == WHALE_NODE_SPECIATION || d.kind == WHALE_NODE_ROOT) {
-        const double e0 = eps_top(M, d.child0), e1 = eps_top(M, d.child1);
-        ebar[d.child0] += g * e1;
-        ebar[d.child1] += g * e0;
-      }
+  // parents before children: ε̄ of a node's row 0 into its children's tops
+  // (row 0 of ε: the product of the children's tops, or the WGD retention map)
+  auto down = [&](int e, const NodeDev& d) {
+    const double g = SL[e] * EB[e] + E0[e];
+    if (d.kind == WHALE_NODE_WGD) {
+      const double qq = M.par[3 * n + d.wgd];
+      EB[d.child0] += g * (2.0 * qq * TOP[d.child0] + (1.0 - qq));
+    } else if (d.kind == WHALE_NODE_SPECIATION || d.kind == WHALE_NODE_ROOT) {
+      EB[d.child0] += g * TOP[d.child1];
+      EB[d.child1] += g * TOP[d.child0];
     }
+  };
+  for (int L = 0; L < n_dlevels; ++L) {
+    if (lv == L) down(me, mine);
+    for (int k = t + (int)blockDim.x; k < n; k += blockDim.x)  // trees of more nodes than lanes
+      if (k >= dlevels[L] && k < dlevels[L + 1]) down(dnodes[k], M.node[dnodes[k]]);
     __syncthreads();
   }
-  if (t == 0) {
-    out[0] = s_total;
-    out[1 + 2 * M.n + M.n_wgd] = s_eta;
+  double* dl = out + 1;
+  double* dm = out + 1 + n;
+  double* dq = out + 1 + 2 * n;
+  for (int e = t; e < n; e += blockDim.x) {
+    const NodeDev& d = M.node[e];
+    const double* dn = M.dnode + (size_t)kDnode * e;
+    const double gt = EB[e];
+    const double ga = dn[8] * gt + acc_in[AL.da + e], gb = dn[9] * gt + acc_in[AL.db + e];
+    dl[e] = d.R > 1 ? ga * dn[0] + gb * dn[2] : 0.0;
+    dm[e] = d.R > 1 ? ga * dn[1] + gb * dn[3] : 0.0;
+    if (d.kind == WHALE_NODE_WGD) {
+      const double ec = TOP[d.child0];
+      dq[d.wgd] = acc_in[AL.q + d.wgd] + (SL[e] * gt + E0[e]) * (ec * ec - ec);
+    }
   }
 }
 
@@ -396,8 +512,16 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(ModelDev M, const double*
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
 }
-__global__ void k_fill_f64(double* p, double v, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
+// k_reset: what an evaluation starts from, in one launch: its tickets, the
+// gradient's accumulators (n_acc 0: none) and the FP32 form's flags and count
+// of flagged families (n_flag 0: none).
+__global__ void k_reset(uint32_t* ticket, int n_ticket, double* acc, int n_acc, uint32_t* flag, int n_flag,
+                        uint32_t* fb) {
+  const int i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+  for (int i = i0; i < n_ticket; i += step) ticket[i] = 0u;
+  for (int i = i0; i < n_acc; i += step) acc[i] = 0.0;
+  for (int i = i0; i < n_flag; i += step) flag[i] = 0u;
+  if (i0 == 0 && n_flag > 0) fb[0] = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -459,30 +583,52 @@ hipError_t launch_mix(hipStream_t st, const MixComp* X, int K, const double* log
 }
 
 hipError_t launch_tables(hipStream_t st, const ModelDev& M, double* eps, double* phi, double* psi, double* pack64,
-                         float* pack32, double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels) {
-  hipLaunchKernelGGL(k_tables, dim3(1), dim3(1024), sizeof(int32_t) * (M.n + 1), st, M, eps, phi, psi, pack64, pack32, dnode,
-                     hlevels, hnodes, n_levels);
+                         float* pack32, double* dnode, const int32_t* hlevels, const int32_t* hnodes, int n_levels,
+                         const int32_t* row_node, double* work) {
+  const size_t lds = tables_work_bytes(M.n, M.tab_rows);
+  if (work) {
+    hipLaunchKernelGGL(k_tables<false>, dim3(1), dim3(1024), 0, st, M, eps, phi, psi, pack64, pack32, dnode, hlevels,
+                       hnodes, n_levels, row_node, work);
+    return hipGetLastError();
+  }
+  if (lds > kTabLds) return hipErrorInvalidValue;
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tables<true>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_tables<true>, dim3(1), dim3(1024), lds, st, M, eps, phi, psi, pack64, pack32, dnode, hlevels,
+                     hnodes, n_levels, row_node, work);
   return hipGetLastError();
 }
 
 hipError_t launch_tail(hipStream_t st, const ModelDev& M, const double* fam_ll, uint32_t n_fam, const double* acc,
-                       double* ebar, const int32_t* dlevels, const int32_t* dnodes, int n_dlevels, int cond,
-                       int with_grad, double* out, const double* n_eff) {
-  hipLaunchKernelGGL(k_tail, dim3(1), dim3(kTailThreads), 0, st, M, fam_ll, n_fam, acc, ebar, dlevels, dnodes,
-                     n_dlevels, cond, with_grad, out, n_eff);
+                       double* work, const int32_t* dlevels, const int32_t* dnodes, int n_dlevels, int cond,
+                       int with_grad, double* out, const double* n_eff, double* host_fam, const uint32_t* fb,
+                       uint32_t* host_fb) {
+  // a workgroup for every 2048 families that go to the host
+  const int grid = host_fam ? (int)std::min<uint32_t>(64, 1 + (n_fam - 1) / 2048) : 1;
+  const size_t lds = tail_work_bytes(M.n);
+  if (!with_grad || lds <= kTailLds)
+    hipLaunchKernelGGL(k_tail<true>, dim3(grid), dim3(kTailThreads), with_grad ? lds : 0, st, M, fam_ll, n_fam, acc,
+                       work, dlevels, dnodes, n_dlevels, cond, with_grad, out, n_eff, host_fam, fb, host_fb);
+  else
+    hipLaunchKernelGGL(k_tail<false>, dim3(grid), dim3(kTailThreads), 0, st, M, fam_ll, n_fam, acc, work, dlevels,
+                       dnodes, n_dlevels, cond, with_grad, out, n_eff, host_fam, fb, host_fb);
   return hipGetLastError();
 }
-
+hipError_t launch_reset(hipStream_t st, uint32_t* ticket, int n_ticket, double* acc, int n_acc, uint32_t* flag,
+                        int n_flag, uint32_t* fb) {
+  const int most = std::max(std::max(n_ticket, n_acc), n_flag);
+  hipLaunchKernelGGL(k_reset, dim3(std::min(64, (most + 255) / 256)), dim3(256), 0, st, ticket, n_ticket, acc, n_acc,
+                     flag, n_flag, fb);
+  return hipGetLastError();
+}
 hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, int n) {
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, p, v, n);
   return hipGetLastError();
 }
 
-hipError_t launch_fill_f64(hipStream_t st, double* p, double v, size_t n) {
-  int grid = (int)std::min<size_t>(1024, (n + 255) / 256 + 1);
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid), dim3(256), 0, st, p, v, n);
-  return hipGetLastError();
-}
 
 // ---------------------------------------------------------------------------
 // k_backtrack: stochastic backtracking of reconciled trees from the stored ℓ

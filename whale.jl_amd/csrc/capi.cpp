@@ -57,14 +57,21 @@ struct DBuf {
   template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
-template <typename T>
-hipError_t upload(DBuf& b, const std::vector<T>& v, hipStream_t st) {
-  hipError_t e = b.alloc(v.size() * sizeof(T));
+template <typename V>
+hipError_t upload(DBuf& b, const V& v, hipStream_t st, bool wait = true) {
+  const size_t n = v.size() * sizeof(v[0]);
+  hipError_t e = b.alloc(n);
   if (e != hipSuccess || v.empty()) return e;
-  e = hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
-  if (e != hipSuccess) return e;
+  e = hipMemcpyAsync(b.p, v.data(), n, hipMemcpyHostToDevice, st);
+  if (e != hipSuccess || !wait) return e;
   return hipStreamSynchronize(st);
 }
+
+// waits for a stream at the end of a scope
+struct StreamWait {
+  hipStream_t st;
+  ~StreamWait() { (void)hipStreamSynchronize(st); }
+};
 
 }  // namespace
 
@@ -689,30 +696,32 @@ int whale_batch_create(whale_model* m, int32_t n_fam, const int64_t* fam_clade_o
     const int rc = ensure_gws(b.get(), nullptr);
     if (rc != WHALE_OK) return rc;
   }
-  HIPCHK(upload(b->fam, P.fam, st));
-  HIPCHK(upload(b->stage, P.stage, st));
-  HIPCHK(upload(b->seg, P.seg, st));
-  HIPCHK(upload(b->run, P.run, st));
-  HIPCHK(upload(b->it_gid, P.it_gid, st));
-  HIPCHK(upload(b->fs4, P.fs4, st));
-  HIPCHK(upload(b->fs2, P.fs2, st));
-  HIPCHK(upload(b->bs4, P.bs4, st));
-  HIPCHK(upload(b->bs2, P.bs2, st));
-  HIPCHK(upload(b->rec_ops, P.rec_ops, st));
-  HIPCHK(upload(b->rec_p, P.rec_p, st));
-  HIPCHK(upload(b->ent_ops, P.ent_ops, st));
-  HIPCHK(upload(b->ent_p, P.ent_p, st));
-  HIPCHK(upload(b->clade_size, P.clade_size, st));
-  HIPCHK(upload(b->split_p, P.split_p, st));
-  HIPCHK(upload(b->lvl_f, P.lvl_f, st));
-  HIPCHK(upload(b->lvl_b, P.lvl_b, st));
-  HIPCHK(upload(b->order, b->order_host, st));
+  // copies queued together: every source lives until the wait below
+  std::vector<uint32_t> so(nc + 1), sg((size_t)split_off[nc]);
+  const StreamWait wait_copies{st};  // also where a copy fails
+  HIPCHK(upload(b->fam, P.fam, st, false));
+  HIPCHK(upload(b->stage, P.stage, st, false));
+  HIPCHK(upload(b->seg, P.seg, st, false));
+  HIPCHK(upload(b->run, P.run, st, false));
+  HIPCHK(upload(b->it_gid, P.it_gid, st, false));
+  HIPCHK(upload(b->fs4, P.fs4, st, false));
+  HIPCHK(upload(b->fs2, P.fs2, st, false));
+  HIPCHK(upload(b->bs4, P.bs4, st, false));
+  HIPCHK(upload(b->bs2, P.bs2, st, false));
+  HIPCHK(upload(b->rec_ops, P.rec_ops, st, false));
+  HIPCHK(upload(b->rec_p, P.rec_p, st, false));
+  HIPCHK(upload(b->ent_ops, P.ent_ops, st, false));
+  HIPCHK(upload(b->ent_p, P.ent_p, st, false));
+  HIPCHK(upload(b->clade_size, P.clade_size, st, false));
+  HIPCHK(upload(b->split_p, P.split_p, st, false));
+  HIPCHK(upload(b->lvl_f, P.lvl_f, st, false));
+  HIPCHK(upload(b->lvl_b, P.lvl_b, st, false));
+  HIPCHK(upload(b->order, b->order_host, st, false));
   {
-    std::vector<uint32_t> so(nc + 1), sg((size_t)split_off[nc]);
     for (int64_t c = 0; c <= nc; ++c) so[c] = (uint32_t)split_off[c];
     for (size_t k = 0; k < sg.size(); ++k) sg[k] = (uint32_t)g1[k] | ((uint32_t)g2[k] << 16);
-    HIPCHK(upload(b->spl_off, so, st));
-    HIPCHK(upload(b->spl_g, sg, st));
+    HIPCHK(upload(b->spl_off, so, st, false));
+    HIPCHK(upload(b->spl_g, sg, st, false));
   }
   b->n_rec = P.rec_ops.size();
 
@@ -726,10 +735,11 @@ int whale_batch_create(whale_model* m, int32_t n_fam, const int64_t* fam_clade_o
   HIPCHK(b->ticket.alloc(sizeof(uint32_t) * kTickets));
   HIPCHK(hipHostMalloc((void**)&b->pin_out, sizeof(double) * (3 + 2 * m->h.n + m->h.n_wgd), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void**)&b->pin_fam, sizeof(double) * n_fam, hipHostMallocDefault));
+  HIPCHK(hipStreamSynchronize(st));
   // release host copies the device now owns (keep what ℓ download needs)
-  for (auto* v : {&P.fs4, &P.fs2, &P.bs4, &P.bs2, &P.rec_ops, &P.ent_ops}) std::vector<uint32_t>().swap(*v);
-  std::vector<double>().swap(P.rec_p);
-  std::vector<double>().swap(P.ent_p);
+  for (auto* v : {&P.fs4, &P.fs2, &P.bs4, &P.bs2, &P.rec_ops, &P.ent_ops}) RawVec<uint32_t>().swap(*v);
+  RawVec<double>().swap(P.rec_p);
+  RawVec<double>().swap(P.ent_p);
   *out = b.release();
   return WHALE_OK;
 }

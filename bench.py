@@ -41,15 +41,15 @@ def measured_traffic(kernel):
     workload, from the FETCH_SIZE/WRITE_SIZE profile committed under profiles/
     (copy-calibrated), or None when the profile is absent."""
     path = os.path.join(ROOT, "profiles", "config4_fp32_gradient_hbm_traffic.md")
-    sym = {"k_backward": "`k_backward<float,true,true,false>`",
-           "k_forward": "`k_forward<float,true,true,true,false>`"}[kernel]
+    sym = "| `%s<float," % kernel  # its one-wave and its team launches
+    total = 0.0
     try:
         for line in open(path, encoding="utf-8"):
-            if line.startswith("| " + sym + " |"):
-                return float(line.strip().strip("|").split("|")[-1]) * 1e6
+            if line.startswith(sym):
+                total += float(line.strip().strip("|").split("|")[-1]) * 1e6
     except OSError:
         pass
-    return None
+    return total or None
 
 
 def algorithmic_bytes(st, s_bytes, x_fwd=0, x_bwd=0):

@@ -1,10 +1,10 @@
 // Execution plan of a batch of gene families, shared by the host compiler
-// (host.cpp) and the device kernels (kernels.hip).
+// (host.cpp) and the device kernels (dp.hpp).
 //
 // The reference evaluates one family by walking the species-tree nodes in
 // wm.order and, per node, every compatible clade and every time slice
 // (src/core.jl:31-37, 83-128).  The plan regroups that work for one 64-lane
-// wavefront per family:
+// wavefront, or a team of them, per family:
 //
 //   segment  a (family, node) pair whose compatible-clade set C_e is not
 //            empty; its ℓ block is R_e x |C_e| values, row-major (one row =

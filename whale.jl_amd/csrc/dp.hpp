@@ -1382,6 +1382,12 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
     tsync<Team, Gws>();
     // kRecs entries of a slot from its j0-th: owner, other part, coefficient
     // p·2^(E(γ) + E(other) - E(owner)) (0 past its last)
+    auto scale = [&](uint32_t i, const uint32_t (&o)[kRecs], Real (&c)[kRecs]) WHALE_INLINE {
+      const int Ei = T.E[i];
+#pragma unroll
+      for (int j = 0; j < kRecs; ++j)
+        c[j] = c[j] != Real(0) ? coef_of(c[j], Ei, T.E[o[j] >> 16], T.E[o[j] & 0xffffu]) : Real(0);
+    };
     auto entries = [&](uint32_t x0, uint32_t j0, uint32_t cnt, uint32_t i, uint32_t (&o)[kRecs],
                        Real (&c)[kRecs]) WHALE_INLINE {
 #pragma unroll
@@ -1391,12 +1397,7 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
         o[j] = ent_ops[x];
         c[j] = ok ? (Real)ent_p[x] : Real(0);
       }
-      if (Scaled) {
-        const int Ei = T.E[i];
-#pragma unroll
-        for (int j = 0; j < kRecs; ++j)
-          c[j] = c[j] != Real(0) ? coef_of(c[j], Ei, T.E[o[j] >> 16], T.E[o[j] & 0xffffu]) : Real(0);
-      }
+      if (Scaled) scale(i, o, c);
     };
     // the entries staged for the levels and the pass after them
     if (RS.on) {
@@ -1455,35 +1456,128 @@ __device__ __forceinline__ void bwd_family(const BatchDev& B, const ModelDev& M,
       };
       // d logL / d ℓ of the root's clades, levels from the last (the ubiquitous
       // clade) down: cA Σ c·ā(owner)·ℓ(other) over the splits a clade is a part
-      // of, whose owners are in higher levels
+      // of, whose owners are in higher levels.  FP32 terms that are not in LDS
+      // are read ahead of the chain: a level's first terms during the level
+      // before it, by slot words read another level before.  Reads in the level
+      // itself are three dependent trips to memory, 4400 to 5800 clocks a level
+      // (5000 families 2918 -> 2831 us, 10,000 8666 -> 8572).  FP64 lanes lack
+      // the registers: one family of 240 genes 1372 -> 1427 us.
+      if constexpr (staged || !kF32) {
 #pragma unroll 1
-      for (int L = (int)F.n_lvl - 1; L >= 0; --L) {
-        const uint32_t s0 = LB.at((uint32_t)L), s1 = LB.at((uint32_t)L + 1);
+        for (int L = (int)F.n_lvl - 1; L >= 0; --L) {
+          const uint32_t s0 = LB.at((uint32_t)L), s1 = LB.at((uint32_t)L + 1);
 #pragma unroll 1
-        for (uint32_t k0 = (s0 & ~15u) + wv * kChunk; k0 < s1; k0 += nt) {
-          const uint32_t k = k0 + lane;
-          const bool in = k >= s0 && k < s1;
-          uint32_t z, r0, cnt;
-          slot_of(in ? k : s0, in, z, r0, cnt);
-          const uint32_t i = z & 0xffffu, pos = (z >> 16) & 0xfu;
-          Real t = 0;
+          for (uint32_t k0 = (s0 & ~15u) + wv * kChunk; k0 < s1; k0 += nt) {
+            const uint32_t k = k0 + lane;
+            const bool in = k >= s0 && k < s1;
+            uint32_t z, r0, cnt;
+            slot_of(in ? k : s0, in, z, r0, cnt);
+            const uint32_t i = z & 0xffffu, pos = (z >> 16) & 0xfu;
+            Real t = 0;
 #pragma unroll 1
-          for (uint32_t j0 = 0; __any(j0 < cnt); j0 += kRecs) {
-            uint32_t o[kRecs];
-            Real c[kRecs], a[kRecs], v[kRecs];
-            terms_of(r0, j0, cnt, i, o, c);
+            for (uint32_t j0 = 0; __any(j0 < cnt); j0 += kRecs) {
+              uint32_t o[kRecs];
+              Real c[kRecs], a[kRecs], v[kRecs];
+              terms_of(r0, j0, cnt, i, o, c);
 #pragma unroll
-            for (int j = 0; j < kRecs; ++j) {
-              a[j] = T.A[o[j] & 0xffffu];
-              v[j] = T.V[o[j] >> 16];
+              for (int j = 0; j < kRecs; ++j) {
+                a[j] = T.A[o[j] & 0xffffu];
+                v[j] = T.V[o[j] >> 16];
+              }
+#pragma unroll
+              for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(cA * a[j] * c[j], v[j], t) : t;
             }
-#pragma unroll
-            for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(cA * a[j] * c[j], v[j], t) : t;
+            t = slot_sum(t, pos, slot_steps(pos));
+            if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : t;
           }
-          t = slot_sum(t, pos, slot_steps(pos));
-          if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : t;
+          tsync<Team, Gws>();
         }
-        tsync<Team, Gws>();
+      } else {
+        auto level = [&](uint32_t s0, uint32_t s1, auto&& first) WHALE_INLINE {
+#pragma unroll 1
+          for (uint32_t k0 = (s0 & ~15u) + wv * kChunk; k0 < s1; k0 += nt) {
+            const uint32_t k = k0 + lane;
+            const bool in = k >= s0 && k < s1, lead_chunk = k0 < (s0 & ~15u) + nt;
+            uint32_t z, r0, cnt;
+            uint32_t o[kRecs];
+            Real c[kRecs];
+            if (lead_chunk) {
+              first(z, r0, cnt, o, c);
+              if (!in) z = cnt = 0;
+            } else {
+              slot_of(in ? k : s0, in, z, r0, cnt);
+            }
+            const uint32_t i = z & 0xffffu, pos = (z >> 16) & 0xfu;
+            Real t = 0;
+#pragma unroll 1
+            for (uint32_t j0 = 0; __any(j0 < cnt); j0 += kRecs) {
+              Real a[kRecs], v[kRecs];
+              if (!lead_chunk || j0 > 0) terms_of(r0, j0, cnt, i, o, c);
+              else if (Scaled) scale(i, o, c);
+#pragma unroll
+              for (int j = 0; j < kRecs; ++j) {
+                a[j] = T.A[o[j] & 0xffffu];
+                v[j] = T.V[o[j] >> 16];
+              }
+#pragma unroll
+              for (int j = 0; j < kRecs; ++j) t = j0 + j < cnt ? fma(cA * a[j] * c[j], v[j], t) : t;
+            }
+            t = slot_sum(t, pos, slot_steps(pos));
+            if (z & kSlotLead) T.A[i] = i == n - 1 ? seed : t;
+          }
+          tsync<Team, Gws>();
+        };
+        struct Words {
+          uint32_t z;
+          u2 d;
+        };
+        struct Terms {
+          uint32_t z, r0, cnt, o[kRecs];
+          double p[kRecs];
+        };
+        // of level L (0 below the first): this lane's first slot, its terms
+        auto words = [&](Words& w, int L) WHALE_INLINE {
+          const uint32_t s0 = LB.at((uint32_t)max(L, 0));
+          const uint32_t k = min((s0 & ~15u) + wv * kChunk + lane, ns - 1);
+          w.d = bs2[F.root_bs + k];
+          w.z = bs4[F.root_bs + k].z;
+        };
+        auto terms = [&](Terms& x, const Words& w) WHALE_INLINE {
+          x.z = w.z;
+          x.r0 = w.d.x;
+          x.cnt = w.d.y & 0xffffu;
+#pragma unroll
+          for (int j = 0; j < kRecs; ++j) {
+            const uint32_t y = ent0 + ((uint32_t)j < x.cnt ? x.r0 + j : first);
+            x.o[j] = ent_ops[y];
+            x.p[j] = ent_p[y];
+          }
+        };
+        // level L from x; y takes the terms of the next level from its words,
+        // whose place takes the words of the level after
+        auto step = [&](int L, Terms& x, Terms& y, Words& wy, Words& wx) WHALE_INLINE {
+          terms(y, wy);
+          words(wx, L - 2);
+          level(LB.at((uint32_t)L), LB.at((uint32_t)L + 1),
+                [&](uint32_t& z, uint32_t& r0, uint32_t& cnt, uint32_t(&o)[kRecs], Real(&c)[kRecs]) WHALE_INLINE {
+                  z = x.z, r0 = x.r0, cnt = x.cnt;
+#pragma unroll
+                  for (int j = 0; j < kRecs; ++j) {
+                    o[j] = x.o[j];
+                    c[j] = (uint32_t)j < cnt ? (Real)x.p[j] : Real(0);
+                  }
+                });
+        };
+        Words w0, w1;
+        Terms t0, t1;
+        words(w0, (int)F.n_lvl - 1);
+        words(w1, (int)F.n_lvl - 2);
+        terms(t0, w0);
+#pragma unroll 1
+        for (int L = (int)F.n_lvl - 1; L >= 0; L -= 2) {
+          step(L, t0, t1, w1, w0);
+          if (L > 0) step(L - 1, t1, t0, w0, w1);
+        }
       }
       // With every ā known, all slots at once: with SF = Σ c·ā(owner)·G(other)
       // and SG likewise with F, ī of the tops is cB(ā ε_g + SF), cB(ā ε_f + SG);
